@@ -173,7 +173,6 @@ struct Lds {
   alignas(16) float xres_1[HID];   // two-column pass: position 1's residual stream
   alignas(16) float h1res_1[HID];
   alignas(16) float comb[HID];   // code-predictor frame (workgroup 0): running embedding combine
-  alignas(16) float stage[MAXV];
   uint32_t pen_bits[MAXV / 32];
   int tok[32];
   const bf16_t* embp[16];   // code-predictor embedding tables, loaded once per launch
@@ -444,7 +443,7 @@ constexpr double EPSD = (double)1e-6f;
 // XCDs of 4 workgroups each (workgroup l of the XCD is virtual XCD l & 7 and takes its row groups
 // 8 (l >> 3) .. 8 (l >> 3) + 7, one after another). The exchange slots and their order are those
 // of the batch-1 decomposition, so every stream computes exactly what a batch-1 launch does.
-template <bool BB, bool XL>
+template <bool BB, bool XL, bool SEL>
 __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
   __shared__ Lds s;
   // Accumulation type: f64 in the backbone (its bf16 residual and KV make every stored rounding
@@ -517,7 +516,7 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
   auto tag_of = [&](int lp, int slot) -> uint32_t { return a.tag_base + (uint32_t)(lp * T_NSLOT + slot); };
   // greedy heads (code-predictor groups, the backbone's codec head) select through a two-level
   // exchange of workgroup candidates instead of gathering every logit in one workgroup
-  const bool greedy_sel = !a.sel.do_sample && (BB || a.cp_frame);
+  constexpr bool greedy_sel = !SEL;
   // backbone greedy head with a repetition penalty: the history as a bitmap in LDS (built at launch)
   const bool pen_rows = BB && !a.cp_frame && greedy_sel && a.head != nullptr && a.rep_penalty != 1.0f && SIO(n_history) > 0;
   auto has_head = [&](int pi) -> bool { return a.cp_frame ? pi >= 1 : (a.head != nullptr && pi == a.n_pos - 1); };
@@ -1272,7 +1271,7 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
     const int r = lane >> 4;
     // logits are bf16 values, as the reference's torch.mv over bf16 operands returns them
     // (generator.py:158, :351); ties then go to the lowest id, as torch.argmax
-    if (greedy_sel) {
+    if constexpr (greedy_sel) {
       const int ci0 = row0 + r;
       float cv = -INFINITY;
       if ((lane & 15) == 0 && r < nrows) {
@@ -1312,8 +1311,8 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
     return a.cp_frame ? ld_const(a.cp_heads + (pi - 1)) : a.head;
   };
   // ---- poller: collect a head's logits and select a token
-  auto select = [&](int pi) -> int {
-    if (greedy_sel) {
+  auto select = [&](int pi) QTTS_INLINE -> int {
+    if constexpr (greedy_sel) {
       // Candidates {value, index} are merged by larger value, lower index on ties (an
       // order-independent choice). Level 1: the 128 wave bests of this XCD (L2-local), two per lane.
       const uint32_t tg = a.tag_base + TAG_HEAD + (uint32_t)pi;
@@ -1372,39 +1371,31 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
       bi = __builtin_amdgcn_readfirstlane(bi);
       // a timed-out poll leaves the error word set and may leave garbage: keep the id in range
       return (bi >= 0 && bi < (a.cp_frame ? a.cp_vocab : a.vocab)) ? bi : 0;
-    }
-    const int n = a.cp_frame ? a.cp_vocab : a.vocab;
-    poll_vec_long(P, ws->logits[pi & 1], n, a.tag_base + TAG_HEAD + (uint32_t)pi, s.stage);
-    SelParams sp = a.sel;
-    sp.seed = SIO(seed);
-    if (a.cp_frame) {
-      sp.group = pi;   // CP head pi-1 selects codebook group pi
     } else {
-      // suppress ids [V-1024, V) except EOS (generator.py:71-75)
-      if (a.mask_tail)
-        for (int i = lane; i < n; i += 64)
-          if (i >= n - 1024 && i != a.eos_id) s.stage[i] = -INFINITY;
-      // repetition penalty, once per distinct id (generator.py:161-167)
-      if (a.rep_penalty != 1.0f && SIO(n_history) > 0) {
-        for (int i = lane; i < MAXV / 32; i += 64) s.pen_bits[i] = 0u;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        for (int i = lane; i < SIO(n_history); i += 64) {
-          const int id = SIO(history[i]);
-          if (id >= 0 && id < n) atomicOr(&s.pen_bits[id >> 5], 1u << (id & 31));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        for (int i = lane; i < n; i += 64) {
-          if (s.pen_bits[i >> 5] & (1u << (i & 31))) {
-            const float v = s.stage[i];   // bf16 arithmetic of the reference: the result is rounded to bf16
-            s.stage[i] = rbf(v > 0.f ? v / a.rep_penalty : v * a.rep_penalty);
+      const int n = a.cp_frame ? a.cp_vocab : a.vocab;
+      SelParams sp = a.sel;
+      sp.seed = SIO(seed);
+      sp.group = a.cp_frame ? pi : 0;   // CP head pi-1 selects codebook group pi
+      HeadMask hm = {n, -1, -1, 1.0f};
+      if (!a.cp_frame) {
+        // suppress ids [V-1024, V) except EOS (generator.py:71-75)
+        if (a.mask_tail) hm.tail = n - 1024;
+        hm.eos = a.eos_id;
+        if (a.suppress_eos) hm.drop = a.eos_id;
+        // repetition penalty, once per distinct id (generator.py:161-167)
+        if (a.rep_penalty != 1.0f && SIO(n_history) > 0) {
+          hm.penalty = a.rep_penalty;
+          for (int i = lane; i < MAXV / 32; i += 64) s.pen_bits[i] = 0u;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          for (int i = lane; i < SIO(n_history); i += 64) {
+            const int id = SIO(history[i]);
+            if (id >= 0 && id < n) atomicOr(&s.pen_bits[id >> 5], 1u << (id & 31));
           }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
       }
-      if (a.suppress_eos && a.eos_id >= 0 && a.eos_id < n && lane == 0) s.stage[a.eos_id] = -INFINITY;
-      sp.group = 0;
+      return head_sample<BB>(P, ws_off(P, ws->logits[pi & 1]), n, a.tag_base + TAG_HEAD + (uint32_t)pi, sp, hm, s.pen_bits, &s.sel);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    return wave_select(s.stage, n, sp, &s.sel);
   };
 
   // =====================================================================================
@@ -1887,10 +1878,14 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
 
 #undef SIO
 
-template __global__ void qtts_decode_kernel<true, false>(const KArgs a);
-template __global__ void qtts_decode_kernel<false, false>(const KArgs a);
-template __global__ void qtts_decode_kernel<false, true>(const KArgs a);
-template __global__ void qtts_decode_kernel<true, true>(const KArgs a);
+template __global__ void qtts_decode_kernel<true, false, false>(const KArgs a);
+template __global__ void qtts_decode_kernel<false, false, false>(const KArgs a);
+template __global__ void qtts_decode_kernel<false, true, false>(const KArgs a);
+template __global__ void qtts_decode_kernel<true, true, false>(const KArgs a);
+template __global__ void qtts_decode_kernel<true, false, true>(const KArgs a);
+template __global__ void qtts_decode_kernel<false, false, true>(const KArgs a);
+template __global__ void qtts_decode_kernel<false, true, true>(const KArgs a);
+template __global__ void qtts_decode_kernel<true, true, true>(const KArgs a);
 
 }  // namespace qtts
 
@@ -1946,6 +1941,17 @@ __global__ void zero_kernel(uint4* p, size_t n16) {
     p[i] = make_uint4(0, 0, 0, 0);
 }
 
+// The instantiation of a launch: backbone or code predictor, one stream per XCD or batch 1, and the
+// selection of its heads (sampled or greedy; a launch without a head takes the greedy one).
+const void* decode_fn(bool bb, bool xl, bool sampled) {
+  using namespace qtts;
+  if (sampled)
+    return bb ? (xl ? (const void*)qtts_decode_kernel<true, true, true> : (const void*)qtts_decode_kernel<true, false, true>)
+              : (xl ? (const void*)qtts_decode_kernel<false, true, true> : (const void*)qtts_decode_kernel<false, false, true>);
+  return bb ? (xl ? (const void*)qtts_decode_kernel<true, true, false> : (const void*)qtts_decode_kernel<true, false, false>)
+            : (xl ? (const void*)qtts_decode_kernel<false, true, false> : (const void*)qtts_decode_kernel<false, false, false>);
+}
+
 // gfx950 with 256 CUs, room for one workgroup of every instantiation on each CU (so a launch of
 // 256 workgroups is co-resident when the device is not shared with other kernels), and workgroup
 // b placed on XCC (b + r) % 8 for a fixed rotation r, 32 workgroups per XCD. Every in-kernel wait
@@ -1971,9 +1977,8 @@ hipError_t check_device_locked(int device, DeviceCheck& dc) {
   if (e != hipSuccess) return e;
   if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0 || prop.multiProcessorCount != qtts::NWG)
     return hipErrorInvalidDevice;
-  const void* fns[] = {(const void*)qtts::qtts_decode_kernel<true, false>, (const void*)qtts::qtts_decode_kernel<false, false>,
-                       (const void*)qtts::qtts_decode_kernel<false, true>, (const void*)qtts::qtts_decode_kernel<true, true>};
-  for (const void* fn : fns) {
+  for (int i = 0; i < 8; ++i) {
+    const void* fn = decode_fn(i & 1, i & 2, i & 4);
     int occ = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, qtts::NTHR, 0);
     if (e != hipSuccess || occ < 1) return e != hipSuccess ? e : hipErrorInvalidDevice;
@@ -2051,8 +2056,7 @@ hipError_t launch(bool bb, KArgs& a, hipStream_t stream, bool xl = false, int n_
   a.spin_cap = kSpinCap;
   a.entry_spin_cap = g_entry_cap.load(std::memory_order_relaxed);
   a.trace = g_trace;
-  const void* fn = bb ? (xl ? (const void*)qtts::qtts_decode_kernel<true, true> : (const void*)qtts::qtts_decode_kernel<true, false>)
-                      : (xl ? (const void*)qtts::qtts_decode_kernel<false, true> : (const void*)qtts::qtts_decode_kernel<false, false>);
+  const void* fn = decode_fn(bb, xl, a.sel.do_sample != 0 && (a.head != nullptr || a.cp_frame));
   return ordered_launch(dev, fn, qtts::NTHR, &a, &a.tag_base, a.io[0].ws, n_streams, sizeof(Workspace), stream);
 }
 

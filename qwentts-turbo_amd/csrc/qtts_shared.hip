@@ -155,10 +155,7 @@ struct SLds {
     // 0..7 are the streams; the code-predictor frame's two-column pass puts position 1 of
     // stream s in column 8 + s
     alignas(16) bf16_t xb[3 * XPS];
-    struct {
-      alignas(16) float stage[MAXV];    // token selection of one stream (its own workgroup)
-      SelScratch sel;
-    } z;
+    SelScratch sel;    // token selection of one stream (its own workgroup)
   };
   alignas(16) float red[SWAV][16][2 * NS];   // per wave: its K-slice's partial of 16 rows x 16 columns
   alignas(16) float q[NS][2][HDIM];
@@ -222,14 +219,7 @@ __device__ __forceinline__ bool poll_sum8s(const Poll& P, const uint64_t* p0, ui
 }
 
 
-// Token selection over an LDS logit vector, kept out of line: inlined, the loop-invariant parts of
-// its sampler would be hoisted out of the step loops and hold registers (or spill) for the whole
-// launch; it runs at most once per head.
-__device__ __attribute__((noinline)) int sh_wave_select(const float* lg, int n, SelParams sp, SelScratch* sc) {
-  return wave_select(lg, n, sp, sc);
-}
-
-template <bool BB>
+template <bool BB, bool SEL>
 __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
   __shared__ SLds s;
   // norm statistics in f64 for the backbone (its bf16 residual), f32 in the code predictor
@@ -254,7 +244,7 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
   const TTSLayerWeights* LW = a.layers;
   const int NL = a.num_layers;
   const bool cp = a.cp_frame != 0;
-  const bool cp_greedy = cp && !a.sel.do_sample;
+  const bool cp_greedy = !SEL && cp;
 
   // streams that compute in this launch (the same set in every workgroup): not skipped, and in
   // a code-predictor frame not already at EOS (generator.py:124-125; its done flag is set)
@@ -1189,22 +1179,22 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
     bi = __builtin_amdgcn_readfirstlane(bi);
     return (bi >= 0 && bi < a.cp_vocab) ? bi : 0;   // a timed-out poll may leave garbage
   };
-  // the stream's whole logit vector into LDS, then mask, penalty and wave_select (its own
-  // workgroup only: the selection scratch overlays the projection inputs)
+  // the stream's whole logit vector, masked and penalised, greedy or drawn from (its own workgroup
+  // only: the selection scratch overlays the projection inputs)
   auto select_full = [&](int pi) -> int {
     const int n = cp ? a.cp_vocab : a.vocab;
-    poll_vec_long(P, &ws->logits[pi & 1][wv][0], n, a.tag_base + TAG_HEAD + (uint32_t)pi, s.z.stage);
     SelParams sp = a.sel;
     sp.seed = IO->seed;
-    if (cp) {
-      sp.group = pi;   // CP head pi-1 selects codebook group pi
-    } else {
+    sp.group = cp ? pi : 0;   // CP head pi-1 selects codebook group pi
+    HeadMask hm = {n, -1, -1, 1.0f};
+    if (!cp) {
       // suppress ids [V-1024, V) except EOS (generator.py:71-75)
-      if (a.mask_tail)
-        for (int i = lane; i < n; i += 64)
-          if (i >= n - 1024 && i != a.eos_id) s.z.stage[i] = -INFINITY;
+      if (a.mask_tail) hm.tail = n - 1024;
+      hm.eos = a.eos_id;
+      if (a.suppress_eos) hm.drop = a.eos_id;
       // repetition penalty, once per distinct id, bf16 arithmetic (generator.py:161-167)
       if (a.rep_penalty != 1.0f && IO->n_history > 0) {
+        hm.penalty = a.rep_penalty;
         for (int i = lane; i < MAXV / 32; i += 64) s.pen_bits[wv][i] = 0u;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         for (int i = lane; i < IO->n_history; i += 64) {
@@ -1212,18 +1202,11 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
           if (id >= 0 && id < n) atomicOr(&s.pen_bits[wv][id >> 5], 1u << (id & 31));
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        for (int i = lane; i < n; i += 64) {
-          if (s.pen_bits[wv][i >> 5] & (1u << (i & 31))) {
-            const float v = s.z.stage[i];
-            s.z.stage[i] = rbf(v > 0.f ? v / a.rep_penalty : v * a.rep_penalty);
-          }
-        }
       }
-      if (a.suppress_eos && a.eos_id >= 0 && a.eos_id < n && lane == 0) s.z.stage[a.eos_id] = -INFINITY;
-      sp.group = 0;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    return sh_wave_select(s.z.stage, n, sp, &s.z.sel);
+    const uint32_t off = ws_off(P, &ws->logits[pi & 1][wv][0]), tag = a.tag_base + TAG_HEAD + (uint32_t)pi;
+    if constexpr (SEL) return head_sample<BB>(P, off, n, tag, sp, hm, s.pen_bits[wv], &s.sel);
+    else return head_argmax<BB>(P, off, n, tag, hm, s.pen_bits[wv]);
   };
 
   // =========================================================================================
@@ -1565,7 +1548,7 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
       }
       if (cp) {
         int tok = 0;
-        if (cp_greedy) {
+        if constexpr (!SEL) {
           if (me) tok = select_greedy(pi);
         } else {
           // sampled: the stream's own workgroup selects and publishes the id; every workgroup
@@ -1598,9 +1581,11 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
           if (me && !last_pos) cp_prep_input0(pi + 1, iss);
           else iss();
         }
-      } else if (me && wg == wv) {
-        const int t = select_full(pi);
-        if (lane == 0 && IO->out_token) *IO->out_token = t;
+      } else if constexpr (BB) {
+        if (me && wg == wv) {
+          const int t = select_full(pi);
+          if (lane == 0 && IO->out_token) *IO->out_token = t;
+        }
       }
       stamp(2 + wv);
       ++nstep;
@@ -1635,8 +1620,10 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
   }
 }
 
-template __global__ void qtts_shared_kernel<true>(const SArgs a);
-template __global__ void qtts_shared_kernel<false>(const SArgs a);
+template __global__ void qtts_shared_kernel<true, false>(const SArgs a);
+template __global__ void qtts_shared_kernel<false, false>(const SArgs a);
+template __global__ void qtts_shared_kernel<true, true>(const SArgs a);
+template __global__ void qtts_shared_kernel<false, true>(const SArgs a);
 
 }  // namespace sh
 }  // namespace qtts
@@ -1790,7 +1777,7 @@ hipError_t qtts_backbone_step_shared(int n_streams, void* workspace, const TTSLa
     io.skip = in.skip_if;
   }
   assign_units(a);
-  return qtts_host::launch_persistent((const void*)qtts::sh::qtts_shared_kernel<true>, qtts::sh::STHR, &a, &a.tag_base,
+  return qtts_host::launch_persistent(a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<true, true> : (const void*)qtts::sh::qtts_shared_kernel<true, false>, qtts::sh::STHR, &a, &a.tag_base,
                                       workspace, 1, sizeof(SWorkspace), stream);
 }
 
@@ -1839,7 +1826,7 @@ hipError_t qtts_cp_frame_shared(int n_streams, void* workspace, const CPLayerWei
     io.done = done + st;
     io.seed = sampling ? sampling->seed + (uint64_t)st : 0;
   }
-  return qtts_host::launch_persistent((const void*)qtts::sh::qtts_shared_kernel<false>, qtts::sh::STHR, &a, &a.tag_base,
+  return qtts_host::launch_persistent(a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<false, true> : (const void*)qtts::sh::qtts_shared_kernel<false, false>, qtts::sh::STHR, &a, &a.tag_base,
                                       workspace, 1, sizeof(SWorkspace), stream);
 }
 
