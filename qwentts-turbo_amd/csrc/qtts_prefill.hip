@@ -8,7 +8,9 @@
 // (generator.py:245-257, megakernel_backbone.py:285-294); the first group-0 token comes from
 // the last position's hidden through the codec head (generator.py:113-117). Every value is
 // rounded where that bf16 forward rounds it:
-//   xn  = bf16(w * bf16(x * (1 / sqrt(mean(x^2) + eps))))              RMSNorm (:59-64)
+//   xn  = w x / sqrt(mean(x^2) + eps)                                  RMSNorm (:59-64), as bf16(x w) into
+//         the next product and 1 / sqrt(..) on its f32 sums (one rounding of xn; transformers has two);
+//         the q/k norms and the final norm round as transformers does
 //   q,k,v = bf16(W xn); q,k per head through RMSNorm, then
 //   rope = bf16(bf16(q * cos) + bf16(rotate_half(q) * sin))            bf16 cos/sin tables
 //   s   = scale * (q . k) in f32; att = bf16((sum_j bf16(e^(s_j - m)) v_j) / sum_j e^(s_j - m))
@@ -20,28 +22,17 @@
 // The f32 sums run in MFMA order rather than the CPU's, so an f32 result can land on the other
 // side of a bf16 rounding boundary now and then; parity is a tolerance, not bit equality.
 //
-// Kernels (the host loop over layers is in qtts_backbone_prefill below):
-//   rmsnorm_kernel   one wave per token
-//   gemm_rows_kernel C = A W^T for prompts of at most 128 tokens: all rows in one workgroup, a
-//                    32-row weight slice, operands straight into registers (the token operand
-//                    in the token-fragment layout its producers write), 4 waves splitting K
-//   gemm_dma_kernel  C = A W^T from 256 rows on: 128 x 128 tiles (2 x 2 waves of 64 x 64),
-//                    K steps of 64 copied global -> LDS by DMA through 2-3 swizzled stages
-//   gemm_kernel      C = A W^T for 129-255 rows and the codec head: 128 x 64 tiles (4 waves,
-//                    each 32 rows x 2 MFMA 32x32x16 blocks), K steps of 128, LDS double buffer
-//                    + 2 register stages of branch-free loads
-//                    All three: split-K over grid.z when the tile grid alone would leave CUs
-//                    idle (partials in f32, summed in a fixed order by the reductions);
-//                    epilogues: store, residual add, SwiGLU
-//   rope_kv_kernel   q/k RMSNorm + interleaved mRoPE, K/V cache write, one workgroup per token
-//                    (fused into the split-K reduction of QKV when split: reduce_rope_kernel)
-//   reduce_resid_norm_kernel  split-K O / down: sums, residual add and the next RMSNorm per token
+// Kernels (the host loop over layers is in qtts_backbone_prefill below), five launches a layer:
+//   embed_kernel       the embeddings into the residual stream, layer 0's norm inputs
+//   tile_gemm_kernel   the four projections, K unsplit, with the norms, RoPE, K/V write, residual and SwiGLU
+//                      in their epilogues
 //   attn_kernel      causal GQA, 4 waves per (32-query block, query head) splitting the key
 //                    blocks: S^T = K Q^T on MFMA (each lane then holds one query's scores, so
 //                    the row max and sum stay in the lane and its partner half-wave), one pass
 //                    with a running max, O^T += V^T P^T on MFMA with V^T read from the row-major
 //                    V block through LDS transpose reads, partials merged in wave order
-//   select_kernel    suppress mask + EOS suppression + the decode kernels' wave_select
+//   final_head_kernel  the last token's final norm and codec head
+//   select_kernel      suppress mask + EOS suppression + the decode kernels' selection
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cstddef>
@@ -58,44 +49,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float EPS = 1e-6f;                 // Qwen3RMSNorm eps (config rms_norm_eps)
-constexpr int BM = 128;                      // GEMM tile rows (columns TN: 64 or 128)
-constexpr int GT = 256;                      // GEMM threads (4 waves)
-// K step of a TN-column tile: 128 for the 64-column (small-M, latency-bound) tiles, whose short
-// K loops then take half the load round trips; 64 for the 128-column tiles
-template <int TN> constexpr int bk_of() { return TN == 64 ? 128 : 64; }  // 128-column tiles: gemm_dma_kernel
-constexpr int QKVW = 4096;                   // q | k | v row of one token
 constexpr int QROW = 136;                    // LDS row of the query block: 128 dims + 16-byte pad
-constexpr int MAX_SPLIT = 16;
-
-enum WMode { W_DIRECT, W_QKV, W_O, W_GU, W_DOWN };
-enum Epi { E_STORE, E_RESID, E_SWIGLU };
-
-struct GemmArgs {
-  const bf16_t* A;                 // [M, K] activations, row stride lda
-  int lda;
-  const TTSLayerWeights* layers;   // device table (W_QKV .. W_DOWN)
-  int layer;
-  const bf16_t* B;                 // W_DIRECT: [N, K]
-  int M, N, K;                     // N: virtual columns (SwiGLU: gate/up interleaved by 32)
-  int kchunk;                      // K range per split (grid.z splits)
-  bf16_t* out;
-  int ldo;
-  const bf16_t* res;               // E_RESID: residual (may alias out)
-  int ldr;
-  float* part;                     // split-K partials [splits][M][N]
-};
-
-// What the QKV GEMM needs to finish a head itself (q/k RMSNorm, RoPE, the K/V cache write);
-// kc == nullptr: plain store
-struct RopeArgs {
-  const bf16_t* cos_t;
-  const bf16_t* sin_t;
-  const int* pos3;                 // [3][M] (t, h, w) table rows, or nullptr: row = p0 + token
-  int p0;
-  bf16_t* kc;
-  bf16_t* vc;
-  int max_seq;
-};
 
 __device__ __forceinline__ bf16x8 as_bf8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -108,16 +62,9 @@ __device__ __forceinline__ uint32_t pack_bh(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// Token-fragment layout of the row GEMM's token operand (a [rows][K] bf16 matrix of at most RM
-// rows, K a multiple of 32, rows allocated in whole 16-row blocks): element (m, k) sits where
-// lane (m & 15) + 16 ((k >> 3) & 3) of fragment (m >> 4, k >> 5) holds it in the
-// v_mfma_f32_16x16x32_bf16 B operand. A fragment is 64 x 16 contiguous bytes, so the GEMM reads it
-// with one fully coalesced load. (Rows of 16 lanes on 16 different rows cost the address unit
-// four times the cycles of the same bytes in contiguous order.) Eight consecutive k of one row stay
-// together.
-__device__ __forceinline__ size_t frag_at(int m, int k, int K) {
-  return ((((size_t)(m >> 4) * (K >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (m & 15)) << 3) + (k & 7);
-}
+#define QTTS_PF_INLINE __attribute__((always_inline))
+typedef __attribute__((address_space(1))) void gvoid_t;
+typedef __attribute__((address_space(3))) void lvoid_t;
 
 __device__ __forceinline__ const bf16_t* tbl(const TTSLayerWeights* lw, int field) {
   return reinterpret_cast<const bf16_t*>(ld_const(reinterpret_cast<const void* const*>(lw) + field));
@@ -129,826 +76,59 @@ __device__ __forceinline__ float silu_f(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
 
-template <int EPI>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, int m, int n, float v) {
-  if constexpr (EPI == E_STORE) {
-    g.out[(size_t)m * g.ldo + n] = f2bh(v);
-  } else if constexpr (EPI == E_RESID) {
-    const float r = bf2f(g.res[(size_t)m * g.ldr + n]);
-    g.out[(size_t)m * g.ldo + n] = f2bh(r + rbh(v));
+// The last token's final norm (hidden, bf16 values as f32) and, with a codec head, its logits: every wave
+// norms the row for itself (2 KB) and takes RPW rows of the head. One launch; as a norm, a split-K matrix
+// product and its reduction it took three, 14 us together.
+constexpr int RPW = 4;
+__global__ void __launch_bounds__(256) final_head_kernel(const bf16_t* x, const bf16_t* gain, const bf16_t* head, int vocab,
+                                                         float* out_hidden, bf16_t* logits) {
+  const int lane = threadIdx.x & 63, w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  u32x4 v[2], gw[2], hw[RPW][2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    v[k] = ldw(x + 8 * (lane + 64 * k));
+    gw[k] = ldw(gain + 8 * (lane + 64 * k));
   }
-}
-
-// output column j of the SwiGLU GEMM from its gate and up sums
-__device__ __forceinline__ void epilogue_swiglu(const GemmArgs& g, int m, int j, float gs, float us) {
-  const float a = rbh(silu_f(rbh(gs)));
-  g.out[(size_t)m * g.ldo + j] = f2bh(a * rbh(us));
-}
-
-// SwiGLU tiles of TN virtual columns hold TN / 2 outputs: rows [64 q, 64 q + 32) of the tile are
-// gate rows and [64 q + 32, 64 q + 64) the up rows of the same 32 outputs, so each wave's two
-// 32-column MFMA blocks are a (gate, up) pair in the same lanes. Virtual column n -> weight row:
-template <int TN>
-__device__ __forceinline__ int swiglu_row(int n, bool& up) {
-  const int tt = n / TN, r = n % TN;
-  up = ((r >> 5) & 1) != 0;
-  return (TN / 2) * tt + 32 * (r >> 6) + (r & 31);
-}
-// ... and output column j -> its gate virtual column (the up column is 32 further)
-template <int TN>
-__device__ __forceinline__ int swiglu_gate_col(int j) {
-  const int tt = j / (TN / 2), r = j % (TN / 2);
-  return TN * tt + 64 * (r >> 5) + (r & 31);
-}
-
-// Weight row of virtual column n of a layer projection (SwiGLU: the tile interleave of swiglu_row)
-template <int WM, int TN>
-__device__ __forceinline__ const bf16_t* weight_row(const GemmArgs& g, const TTSLayerWeights* lw, int n) {
-  if constexpr (WM == W_DIRECT) {
-    return g.B + (size_t)n * g.K;
-  } else if constexpr (WM == W_QKV) {
-    return n < 2048 ? tbl(lw, 1) + (size_t)n * g.K
-                    : (n < 3072 ? tbl(lw, 2) + (size_t)(n - 2048) * g.K : tbl(lw, 3) + (size_t)(n - 3072) * g.K);
-  } else if constexpr (WM == W_O) {
-    return tbl(lw, 6) + (size_t)n * g.K;
-  } else if constexpr (WM == W_GU) {
-    bool up;
-    const int row = swiglu_row<TN>(n, up);
-    return (up ? tbl(lw, 9) : tbl(lw, 8)) + (size_t)row * g.K;
-  } else {
-    return tbl(lw, 10) + (size_t)n * g.K;
+  if (head != nullptr) {
+#pragma unroll
+    for (int r = 0; r < RPW; ++r)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) hw[r][k] = ldw(head + (size_t)min(RPW * w + r, vocab - 1) * HID + 8 * (lane + 64 * k));
   }
-}
-
-// C = A W^T on a BM x 64 tile (prompts of 129-255 tokens, and the codec head): wave w owns rows
-// 32 w .. 32 w + 31 and both 32-column blocks; K steps of 128 through an LDS double buffer fed
-// from register stages.
-template <int WM, int EPI, int TN>
-__global__ void __launch_bounds__(GT, 1) gemm_kernel(const GemmArgs g) {
-  static_assert(TN == 64, "the 128-column tiles run in gemm_dma_kernel");
-  constexpr int BK = bk_of<TN>();
-  constexpr int LROW = BK + 8;                     // LDS row (bf16): 16-byte aligned, skewed banks
-  constexpr int CPR = BK / 8;                      // 16-byte chunks per tile row
-  constexpr int RPP = GT / CPR;                    // tile rows one pass of the workgroup loads
-  constexpr int NAR = BM / RPP;                    // A chunks per thread
-  constexpr int NBR = TN / RPP;                    // B chunks per thread
-  constexpr int MBW = 1;                           // 32-row blocks per wave
-  __shared__ __attribute__((aligned(16))) bf16_t sa[2][BM * LROW];
-  __shared__ __attribute__((aligned(16))) bf16_t sb[2][TN * LROW];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * TN;
-  const int kbeg = blockIdx.z * g.kchunk, nk = g.kchunk / BK;
-  const int lr = t / CPR, lc = (t % CPR) * 8;   // this thread's load row (within RPP) and column
-  const int wr0 = 32 * w, wc0 = 0;                // wave's first tile row and column
-
-  // weight rows this thread stages (virtual columns n0 + lr + 32 i)
-  const bf16_t* brow[NBR];
-  {
-    const TTSLayerWeights* lw = g.layers + g.layer;
-#pragma unroll
-    for (int i = 0; i < NBR; ++i) brow[i] = weight_row<WM, TN>(g, lw, n0 + lr + RPP * i) + kbeg + lc;
-  }
-  const bf16_t* arow[NAR];
-  bool aok[NAR];
-#pragma unroll
-  for (int i = 0; i < NAR; ++i) {
-    const int m = m0 + lr + RPP * i;
-    aok[i] = m < g.M;
-    arow[i] = g.A + (size_t)(aok[i] ? m : 0) * g.lda + kbeg + lc;
-  }
-
-  // NST register stages ahead of the MFMAs (tile kt + NST loads while tile kt computes and tile
-  // kt + 1 moves to LDS). Every load is issued unconditionally (rows past M read row 0 and are
-  // zeroed afterwards; K steps past the end reload the last one): a load under a branch makes the
-  // compiler wait for all outstanding loads instead of just the old ones.
-  constexpr int NST = 2;   // a third stage measured 5-10% slower
-  u32x4 ra[NST][NAR], rb[NST][NBR];
-  auto gload = [&](int k0, u32x4 (&a)[NAR], u32x4 (&b)[NBR]) {
-#pragma unroll
-    for (int i = 0; i < NAR; ++i) {
-      const u32x4 v = ldw(arow[i] + k0);
-      a[i] = aok[i] ? v : u32x4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int i = 0; i < NBR; ++i) b[i] = ldw(brow[i] + k0);
-  };
-  auto sstore = [&](int buf, const u32x4 (&a)[NAR], const u32x4 (&b)[NBR]) {
-#pragma unroll
-    for (int i = 0; i < NAR; ++i) *reinterpret_cast<u32x4*>(&sa[buf][(lr + RPP * i) * LROW + lc]) = a[i];
-#pragma unroll
-    for (int i = 0; i < NBR; ++i) *reinterpret_cast<u32x4*>(&sb[buf][(lr + RPP * i) * LROW + lc]) = b[i];
-  };
-
-  f32x16 acc[MBW][2];
-#pragma unroll
-  for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.0f;
-
-  const int arow_l = (wr0 + (lane & 31)) * LROW, brow_l = (wc0 + (lane & 31)) * LROW, kh = 8 * (lane >> 5);
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const int ko = 16 * kk + kh;
-      bf16x8 av[MBW], bv[2];
-#pragma unroll
-      for (int mb = 0; mb < MBW; ++mb)
-        av[mb] = as_bf8(*reinterpret_cast<const u32x4*>(&sa[buf][arow_l + 32 * mb * LROW + ko]));
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-        bv[nb] = as_bf8(*reinterpret_cast<const u32x4*>(&sb[buf][brow_l + 32 * nb * LROW + ko]));
-#pragma unroll
-      for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-          acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mb], bv[nb], acc[mb][nb], 0, 0, 0);
-    }
-  };
-  // one step: tile kt in LDS buffer kt & 1, tile kt + 1 in register stage (kt + 1) % NST, stage
-  // kt % NST free (its tile went to LDS in the previous step)
-  auto step = [&](int kt, u32x4 (&a0)[NAR], u32x4 (&b0)[NBR], const u32x4 (&a1)[NAR], const u32x4 (&b1)[NBR]) {
-    gload(min(kt + NST, nk - 1) * BK, a0, b0);
-    compute(kt & 1);
-    if (kt + 1 < nk) sstore((kt + 1) & 1, a1, b1);
-    __syncthreads();
-  };
-
-#pragma unroll
-  for (int st = 0; st < NST; ++st) gload(min(st, nk - 1) * BK, ra[st], rb[st]);
-  sstore(0, ra[0], rb[0]);
-  __syncthreads();
-  for (int kt = 0; kt < nk; kt += NST) {
-    step(kt, ra[0], rb[0], ra[1], rb[1]);
-    if (kt + 1 < nk) step(kt + 1, ra[1], rb[1], ra[0], rb[0]);
-  }
-
-  // D layout of a 32x32 block: lane column lane & 31; register r holds row
-  // 8 (r >> 2) + 4 (lane >> 5) + (r & 3)
-  const int col = lane & 31, hrow = 4 * (lane >> 5);
-  if (gridDim.z > 1) {
-    float* P = g.part + (size_t)blockIdx.z * g.M * g.N;
-#pragma unroll
-    for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + wr0 + 32 * mb + 8 * (r >> 2) + hrow + (r & 3);
-          if (m < g.M) P[(size_t)m * g.N + n0 + wc0 + 32 * nb + col] = acc[mb][nb][r];
-        }
-    return;
-  }
-#pragma unroll
-  for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = m0 + wr0 + 32 * mb + 8 * (r >> 2) + hrow + (r & 3);
-      if (m >= g.M) continue;
-      if constexpr (EPI == E_SWIGLU) {
-        epilogue_swiglu(g, m, n0 / 2 + wc0 / 2 + col, acc[mb][0][r], acc[mb][1][r]);
-      } else {
-        epilogue<EPI>(g, m, n0 + wc0 + col, acc[mb][0][r]);
-        epilogue<EPI>(g, m, n0 + wc0 + 32 + col, acc[mb][1][r]);
-      }
-    }
-}
-
-// Token-row GEMM for prompts of at most RM tokens: all M rows in one workgroup, a tile of TN
-// weight rows (virtual columns). At this size the weights are the only large operand (the token
-// rows are at most 256 KB and stay in L2), so the kernel is a weight stream. Each workgroup
-// streams its own slice of the weights, and all the operands go straight into registers in the
-// v_mfma_f32_16x16x32_bf16 layout, with no LDS staging and no barrier in the K loop:
-// - weight block nb is the A operand: lane l holds 8 bf16 of weight row 16 nb + (l & 15) at
-//   k = 32 s + 8 (l >> 4);
-// - token block mb is the B operand: the same for token row 16 mb + (l & 15), read from the
-//   token-fragment layout (frag_at) as one contiguous 1 KB fragment. Blocks past the last row
-//   block read the last one, and the sums of rows past M are never stored.
-// The 4 waves split the workgroup's K range (g.kchunk = 4 x 32 x NST) into quarters. Each wave
-// keeps D steps of loads in flight. The quarter sums meet in LDS and are added in wave order,
-// then go through the GEMM's epilogue, or to the split-K partials when grid.z > 1. A SwiGLU
-// tile's first TN / 2 weight rows are gate rows of outputs TN / 2 x tile + 0 .. TN / 2 - 1, its
-// last TN / 2 the up rows of the same outputs; its output (the down projection's input) is
-// written in the token-fragment layout. This kernel never splits SwiGLU.
-constexpr int RM = 128;
-
-template <int WM, int EPI, int TN, int NST>
-__global__ void __launch_bounds__(GT, 2) gemm_rows_kernel(const GemmArgs g) {
-  static_assert(WM != W_DIRECT && TN % 32 == 0, "row GEMM: layer weights, 16-row blocks in pairs");
-  constexpr int NB = TN / 16, MB = RM / 16;
-  constexpr int D = NST < 4 ? NST : 4;
-  constexpr int RROW = TN + 4;                 // f32 LDS row of a quarter sum (16-byte aligned)
-  __shared__ __attribute__((aligned(16))) float red[4][RM * RROW];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6, i = lane & 15, kg = lane >> 4;
-  const int n0 = blockIdx.x * TN;
-  const int k0 = blockIdx.z * g.kchunk + w * (32 * NST) + 8 * kg;
-  const TTSLayerWeights* lw = g.layers + g.layer;
-  const bf16_t* wp[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    const int n = n0 + 16 * nb + i;
-    const bf16_t* p;
-    if constexpr (WM == W_QKV) {
-      p = n < 2048 ? tbl(lw, 1) + (size_t)n * g.K
-                   : (n < 3072 ? tbl(lw, 2) + (size_t)(n - 2048) * g.K : tbl(lw, 3) + (size_t)(n - 3072) * g.K);
-    } else if constexpr (WM == W_O) {
-      p = tbl(lw, 6) + (size_t)n * g.K;
-    } else if constexpr (WM == W_GU) {
-      const int j = n0 / 2 + 16 * (nb % (NB / 2)) + i;
-      p = (nb < NB / 2 ? tbl(lw, 8) : tbl(lw, 9)) + (size_t)j * g.K;
-    } else {
-      p = tbl(lw, 10) + (size_t)n * g.K;
-    }
-    wp[nb] = p + k0;
-  }
-  const bf16_t* xp[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-    xp[mb] = g.A + (((size_t)min(mb, (g.M - 1) >> 4) * (g.K >> 5) + ((k0 - 8 * kg) >> 5)) * 64 + lane) * 8;
-
-  u32x4 wr[D][NB], xr[D][MB];
-  f32x4 acc[NB][MB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < D; ++s) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) wr[s][nb] = ldw(wp[nb] + 32 * s);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) xr[s][mb] = ldw(xp[mb] + 512 * s);
-  }
-#pragma unroll
-  for (int s = 0; s < NST; ++s) {
-    const int d = s % D;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        acc[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(wr[d][nb]), as_bf8(xr[d][mb]), acc[nb][mb], 0, 0, 0);
-    if (s + D < NST) {   // compile-time after unrolling
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) wr[d][nb] = ldw(wp[nb] + 32 * (s + D));
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) xr[d][mb] = ldw(xp[mb] + 512 * (s + D));
-    }
-  }
-
-  // D layout: lane l holds weight rows 4 (l >> 4) + e of token column l & 15
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      *reinterpret_cast<f32x4*>(&red[w][(16 * mb + i) * RROW + 16 * nb + 4 * kg]) = acc[nb][mb];
-  __syncthreads();
-  auto qsum = [&](int off) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(&red[0][off]);
-    const f32x4 b = *reinterpret_cast<const f32x4*>(&red[1][off]);
-    const f32x4 c = *reinterpret_cast<const f32x4*>(&red[2][off]);
-    const f32x4 e = *reinterpret_cast<const f32x4*>(&red[3][off]);
-    return ((a + b) + c) + e;
-  };
-  if constexpr (EPI == E_SWIGLU) {
-    constexpr int C4 = TN / 8;                 // groups of 4 outputs per token row
-#pragma unroll
-    for (int q = t; q < RM * C4; q += GT) {
-      const int m = q / C4, c = 4 * (q % C4);
-      if (m >= g.M) break;
-      const f32x4 gs = qsum(m * RROW + c), us = qsum(m * RROW + TN / 2 + c);
-      u32x2 o;
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float a0 = rbh(silu_f(rbh(gs[2 * e]))) * rbh(us[2 * e]);
-        const float a1 = rbh(silu_f(rbh(gs[2 * e + 1]))) * rbh(us[2 * e + 1]);
-        o[e] = pack_bh(a0, a1);
-      }
-      *reinterpret_cast<u32x2*>(g.out + frag_at(m, n0 / 2 + c, g.ldo)) = o;
-    }
-  } else {
-    constexpr int C4 = TN / 4;
-#pragma unroll
-    for (int q = t; q < RM * C4; q += GT) {
-      const int m = q / C4, c = 4 * (q % C4);
-      if (m >= g.M) break;
-      const f32x4 v = qsum(m * RROW + c);
-      if (gridDim.z > 1) {
-        *reinterpret_cast<f32x4*>(g.part + (size_t)blockIdx.z * g.M * g.N + (size_t)m * g.N + n0 + c) = v;
-      } else if constexpr (EPI == E_RESID) {
-        const u32x2 r = *reinterpret_cast<const u32x2*>(g.res + (size_t)m * g.ldr + n0 + c);
-        u32x2 o;
-        o[0] = pack_bh(bflo(r[0]) + rbh(v[0]), bfhi(r[0]) + rbh(v[1]));
-        o[1] = pack_bh(bflo(r[1]) + rbh(v[2]), bfhi(r[1]) + rbh(v[3]));
-        *reinterpret_cast<u32x2*>(g.out + (size_t)m * g.ldo + n0 + c) = o;
-      } else {
-        u32x2 o;
-        o[0] = pack_bh(v[0], v[1]);
-        o[1] = pack_bh(v[2], v[3]);
-        *reinterpret_cast<u32x2*>(g.out + (size_t)m * g.ldo + n0 + c) = o;
-      }
-    }
-  }
-}
-
-#define QTTS_PF_INLINE __attribute__((always_inline))
-typedef __attribute__((address_space(1))) void gvoid_t;
-typedef __attribute__((address_space(3))) void lvoid_t;
-
-// C = A W^T on a 128 x 128 tile (prompts from 256 tokens on), K steps of 64, with the operands
-// copied from global memory straight into LDS (global_load_lds_dwordx4: each wave instruction
-// writes 64 x 16 bytes at a wave-uniform LDS address) through NS stages. No register staging and
-// no LDS store instructions; one barrier per K step.
-// - LDS tile layout: row r of a stage holds its 8 16-byte k-chunks with chunk c at position
-//   c ^ (r & 7). A DMA instruction covers 8 rows; lane l writes position l & 7 of row l >> 3 and
-//   so loads chunk (l & 7) ^ (r & 7) of that row: 8 lanes read one 128-byte row segment.
-// - The XOR swizzle makes the MFMA operand reads (32 rows at one chunk) conflict-free.
-// - Waves form 2 x 2; wave w owns rows 64 (w & 1) .. + 63 and columns 64 (w >> 1) .. + 63 (two
-//   32 x 32 MFMA blocks each way), as in gemm_kernel's 128-column tile, and the epilogues match.
-// - Rows past M read row M - 1; their sums are never stored.
-// - The wait before each barrier counts this wave's DMA instructions still in flight: the
-//   compiler does not track LDS writes made by DMA.
-// - Unsplit QKV with rope arguments: a tile is one head of 128 tokens, and the epilogue finishes
-//   it as rope_kv_apply does: bf16 tile through LDS, then two threads per token (32 channel pairs
-//   (d, d + 64) each) for the q/k RMSNorm and the interleaved mRoPE. q goes back to the QKV rows;
-//   k and v go to the cache.
-template <int WM, int EPI, int NS>
-__global__ void __launch_bounds__(GT, NS <= 2 ? 2 : 1) gemm_dma_kernel(const GemmArgs g, const RopeArgs ra) {
-  constexpr int TN = 128, TM = 128, BK = 64;
-  constexpr int STAGE = (TM + TN) * BK * 2;        // bytes of one stage (A then B)
-  constexpr int NIA = TM * BK * 2 / 1024 / 4;      // DMA instructions per wave for A (4)
-  constexpr int NIB = TN * BK * 2 / 1024 / 4;      // ... and for B (4)
-  constexpr int NIW = NIA + NIB;
-  static_assert(NS >= 2 && NS <= 4 && NIW <= 15, "stages / vmcnt field");
-  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int kbeg = blockIdx.z * g.kchunk, nk = g.kchunk / BK;
-  const TTSLayerWeights* lw = g.layers + g.layer;
-
-  // this lane's source rows: instruction i of the wave covers tile rows 8 (NIA w + i) .. + 7
-  const bf16_t* asrc[NIA];
-  const bf16_t* bsrc[NIB];
-#pragma unroll
-  for (int i = 0; i < NIA; ++i) {
-    const int r = 8 * (NIA * w + i) + (lane >> 3);
-    const int c = (lane & 7) ^ (r & 7);
-    asrc[i] = g.A + (size_t)min(m0 + r, g.M - 1) * g.lda + kbeg + 8 * c;
-  }
-#pragma unroll
-  for (int i = 0; i < NIB; ++i) {
-    const int r = 8 * (NIB * w + i) + (lane >> 3);
-    const int c = (lane & 7) ^ (r & 7);
-    bsrc[i] = weight_row<WM, TN>(g, lw, n0 + r) + kbeg + 8 * c;
-  }
-  // stage s <- K step kt (clamped: steps past the end reload the last one)
-  auto issue = [&](int s, int kt) QTTS_PF_INLINE {
-    const int k = BK * min(kt, nk - 1);
-    char* base = lds + s * STAGE;
-#pragma unroll
-    for (int i = 0; i < NIA; ++i)
-      __builtin_amdgcn_global_load_lds((gvoid_t*)(asrc[i] + k), (lvoid_t*)(base + 1024 * (NIA * w + i)), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < NIB; ++i)
-      __builtin_amdgcn_global_load_lds((gvoid_t*)(bsrc[i] + k), (lvoid_t*)(base + TM * BK * 2 + 1024 * (NIB * w + i)),
-                                       16, 0, 0);
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.0f;
-  const int wr0 = 64 * (w & 1), wc0 = 64 * (w >> 1), hk = lane >> 5;
-  // byte offset of (row r, chunk c) in a stage's A or B part
-  auto at = [](int r, int c) { return (r * 8 + (c ^ (r & 7))) * 16; };
-  auto compute = [&](int s) QTTS_PF_INLINE {
-    const char* a = lds + s * STAGE;
-    const char* b = a + TM * BK * 2;
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const int c = 2 * kk + hk;
-      bf16x8 av[2], bv[2];
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb) av[mb] = as_bf8(*reinterpret_cast<const u32x4*>(a + at(wr0 + 32 * mb + (lane & 31), c)));
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb) bv[nb] = as_bf8(*reinterpret_cast<const u32x4*>(b + at(wc0 + 32 * nb + (lane & 31), c)));
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-          acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mb], bv[nb], acc[mb][nb], 0, 0, 0);
-    }
-  };
-
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s) issue(s, s);
-  for (int kt = 0; kt < nk; ++kt) {
-    // this wave's DMA for step kt has landed when at most (NS - 2) stages' instructions remain
-    __builtin_amdgcn_s_waitcnt(0x0F70 | ((NS - 2) * NIW));
-    __builtin_amdgcn_s_barrier();   // every wave's step kt is in LDS; step kt - 1's buffer is free
-    issue((kt + NS - 1) % NS, kt + NS - 1);
-    compute(kt % NS);
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // no DMA may still target LDS when the workgroup ends
-
-  const int col = lane & 31, hrow = 4 * (lane >> 5);
-  if constexpr (WM == W_QKV && EPI == E_STORE) {
-    if (ra.kc != nullptr) {
-      constexpr int TR = HDIM + 8;   // bf16 row of the staged head tile (16-byte aligned, skewed)
-      bf16_t* T = reinterpret_cast<bf16_t*>(lds);
-      __syncthreads();   // every wave's DMA has landed and its last MFMA reads are done
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            T[(wr0 + 32 * mb + 8 * (r >> 2) + hrow + (r & 3)) * TR + wc0 + 32 * nb + col] = f2bh(acc[mb][nb][r]);
-      __syncthreads();
-      const int head = n0 / HDIM;   // q heads 0..15, k heads 16..23, v heads 24..31
-      if (head >= NQH + NKVH) {
-        bf16_t* vbase = ra.vc + ((size_t)g.layer * NKVH + (head - NQH - NKVH)) * ra.max_seq * HDIM;
-        for (int q = t; q < TM * 16; q += GT) {
-          const int row = q >> 4, ch = 8 * (q & 15), m = m0 + row;
-          if (m < g.M)
-            *reinterpret_cast<u32x4*>(vbase + (size_t)(ra.p0 + m) * HDIM + ch) =
-                *reinterpret_cast<const u32x4*>(&T[row * TR + ch]);
-        }
-        return;
-      }
-      const int row = t >> 1, hf = t & 1, m = min(m0 + row, g.M - 1);
-      const bf16_t* tr = &T[row * TR + 32 * hf];
-      float ss = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(tr + 8 * c);
-        const u32x4 b = *reinterpret_cast<const u32x4*>(tr + 64 + 8 * c);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          ss += bflo(a[e]) * bflo(a[e]) + bflo(b[e]) * bflo(b[e]);
-          ss += bfhi(a[e]) * bfhi(a[e]) + bfhi(b[e]) * bfhi(b[e]);
-        }
-      }
-      ss += __shfl_xor(ss, 1, 64);
-      const float rs = 1.0f / sqrtf(ss / (float)HDIM + EPS);
-      const bool isq = head < NQH;
-      const bf16_t* gn = tbl(lw, isq ? 4 : 5);
-      // table rows of the three sections (t, h, w); channel d < 60 takes h when d % 3 == 1 and w
-      // when d % 3 == 2, every other channel t (the same row for d and d + 64)
-      const int pos = ra.p0 + m;
-      int rsec[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) rsec[j] = ra.pos3 ? min(max(ra.pos3[j * g.M + m], 0), ra.max_seq - 1) : pos;
-      bf16_t* dst = isq ? g.out + (size_t)m * g.ldo + n0
-                        : ra.kc + (((size_t)g.layer * NKVH + (head - NQH)) * ra.max_seq + pos) * HDIM;
-      // 8 channel pairs (d0 + e, d0 + 64 + e); cs/sn: this chunk's cos and sin for d and d + 64,
-      // already picked per section
-      auto finish = [&](int c, const float (&c0)[8], const float (&c1)[8], const float (&s0)[8],
-                        const float (&s1)[8], const u32x4& g0, const u32x4& g1) QTTS_PF_INLINE {
-        const int d0 = 32 * hf + 8 * c;
-        const u32x4 a = *reinterpret_cast<const u32x4*>(tr + 8 * c);
-        const u32x4 b = *reinterpret_cast<const u32x4*>(tr + 64 + 8 * c);
-        u32x4 o0, o1;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float r0[2], r1[2];
-#pragma unroll
-          for (int h2 = 0; h2 < 2; ++h2) {
-            const int k = 2 * e + h2;
-            const float x0 = h2 ? bfhi(a[e]) : bflo(a[e]), x1 = h2 ? bfhi(b[e]) : bflo(b[e]);
-            const float ga = h2 ? bfhi(g0[e]) : bflo(g0[e]), gb = h2 ? bfhi(g1[e]) : bflo(g1[e]);
-            const float y0 = rbh(ga * rbh(x0 * rs)), y1 = rbh(gb * rbh(x1 * rs));
-            r0[h2] = rbh(y0 * c0[k]) + rbh(-y1 * s0[k]);
-            r1[h2] = rbh(y1 * c1[k]) + rbh(y0 * s1[k]);
-          }
-          o0[e] = pack_bh(r0[0], r0[1]);
-          o1[e] = pack_bh(r1[0], r1[1]);
-        }
-        if (m0 + row < g.M) {
-          *reinterpret_cast<u32x4*>(dst + d0) = o0;
-          *reinterpret_cast<u32x4*>(dst + d0 + 64) = o1;
-        }
-      };
-      auto unpack8 = [](const u32x4& v, float (&f)[8]) QTTS_PF_INLINE {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { f[2 * e] = bflo(v[e]); f[2 * e + 1] = bfhi(v[e]); }
-      };
-      if (ra.pos3 == nullptr) {
-        // one table row per token: every load of the 4 chunks issued before the first use
-        const bf16_t* cr = ra.cos_t + (size_t)pos * HDIM + 32 * hf;
-        const bf16_t* sr = ra.sin_t + (size_t)pos * HDIM + 32 * hf;
-        u32x4 vc0[4], vc1[4], vs0[4], vs1[4], vg0[4], vg1[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          vc0[c] = ldw(cr + 8 * c); vc1[c] = ldw(cr + 64 + 8 * c);
-          vs0[c] = ldw(sr + 8 * c); vs1[c] = ldw(sr + 64 + 8 * c);
-          vg0[c] = ldw(gn + 32 * hf + 8 * c); vg1[c] = ldw(gn + 64 + 32 * hf + 8 * c);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          float c0[8], c1[8], s0[8], s1[8];
-          unpack8(vc0[c], c0); unpack8(vc1[c], c1); unpack8(vs0[c], s0); unpack8(vs1[c], s1);
-          finish(c, c0, c1, s0, s1, vg0[c], vg1[c]);
-        }
-      } else {
-#pragma unroll 1
-        for (int c = 0; c < 4; ++c) {
-          const int d0 = 32 * hf + 8 * c;
-          u32x4 cs0[3], cs1[3], sn0[3], sn1[3];
-#pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            const size_t ro = (size_t)rsec[j] * HDIM + d0;
-            cs0[j] = ldw(ra.cos_t + ro); cs1[j] = ldw(ra.cos_t + ro + 64);
-            sn0[j] = ldw(ra.sin_t + ro); sn1[j] = ldw(ra.sin_t + ro + 64);
-          }
-          float c0[8], c1[8], s0[8], s1[8];
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const int d = d0 + k, sec = (d < 60 && d % 3 == 1) ? 1 : ((d < 60 && d % 3 == 2) ? 2 : 0);
-            auto pick = [&](const u32x4 (&v)[3]) {
-              const uint32_t wv = sec == 0 ? v[0][k >> 1] : (sec == 1 ? v[1][k >> 1] : v[2][k >> 1]);
-              return (k & 1) ? bfhi(wv) : bflo(wv);
-            };
-            c0[k] = pick(cs0); c1[k] = pick(cs1); s0[k] = pick(sn0); s1[k] = pick(sn1);
-          }
-          finish(c, c0, c1, s0, s1, ldw(gn + d0), ldw(gn + d0 + 64));
-        }
-      }
-      return;
-    }
-  }
-  if (gridDim.z > 1) {
-    float* P = g.part + (size_t)blockIdx.z * g.M * g.N;
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + wr0 + 32 * mb + 8 * (r >> 2) + hrow + (r & 3);
-          if (m < g.M) P[(size_t)m * g.N + n0 + wc0 + 32 * nb + col] = acc[mb][nb][r];
-        }
-    return;
-  }
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = m0 + wr0 + 32 * mb + 8 * (r >> 2) + hrow + (r & 3);
-      if (m >= g.M) continue;
-      if constexpr (EPI == E_SWIGLU) {
-        epilogue_swiglu(g, m, n0 / 2 + wc0 / 2 + col, acc[mb][0][r], acc[mb][1][r]);
-      } else {
-        epilogue<EPI>(g, m, n0 + wc0 + col, acc[mb][0][r]);
-        epilogue<EPI>(g, m, n0 + wc0 + 32 + col, acc[mb][1][r]);
-      }
-    }
-}
-
-// Sums in split order of the partials at p + z stride, z < splits: 4 NQ consecutive floats
-// (NQ 16-byte loads per split). The loads go out in groups of G splits before any of them is
-// added (each clamped to the last split, so an unconditional load from a valid address): the
-// group's round trips overlap, where a rolled loop waits for each load before it issues the next.
-// The additions run in split order, so the sums are the ones of a plain loop, bit for bit.
-template <int G, int NQ>
-__device__ __forceinline__ void sum_splits(const float* p, size_t stride, int splits, float (&s)[4 * NQ]) {
-#pragma unroll
-  for (int i = 0; i < 4 * NQ; ++i) s[i] = 0.0f;
-  for (int z0 = 0; z0 < splits; z0 += G) {
-    u32x4 v[G][NQ];
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-        v[j][q] = *reinterpret_cast<const u32x4*>(p + (size_t)min(z0 + j, splits - 1) * stride + 4 * q);
-    // every load of the group is issued here: the compiler may not sink one into a later branch
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(v[j][q]));
-    // a clamped duplicate adds -0.0, the exact identity of IEEE addition, so the sum is the one of
-    // the valid splits alone
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      const bool ok = z0 + j < splits;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[4 * q + e] += ok ? __uint_as_float(v[j][q][e]) : -0.0f;
-    }
-  }
-}
-
-// Sum of the split-K partials in split order, then the GEMM's epilogue; four consecutive
-// outputs per thread (16-byte partial loads; a SwiGLU group of four lies in one 32-column block).
-template <int EPI, int TN>
-__global__ void __launch_bounds__(256) reduce_kernel(const GemmArgs g, int splits) {
-  const int nout = EPI == E_SWIGLU ? g.N / 2 : g.N;
-  const long idx = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (idx >= (long)g.M * nout) return;
-  const int m = (int)(idx / nout), j = (int)(idx % nout);
-  const size_t stride = (size_t)g.M * g.N;
-  const float* P = g.part + (size_t)m * g.N;
-  if constexpr (EPI == E_SWIGLU) {
-    const int nv = swiglu_gate_col<TN>(j);
-    float gs[4], us[4];
-    sum_splits<4, 1>(P + nv, stride, splits, gs);
-    sum_splits<4, 1>(P + nv + 32, stride, splits, us);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) epilogue_swiglu(g, m, j + e, gs[e], us[e]);
-  } else {
-    float v[4];
-    sum_splits<4, 1>(P + j, stride, splits, v);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) epilogue<EPI>(g, m, j + e, v[e]);
-  }
-}
-
-// RMSNorm of M token rows (row stride ldx) into bf16 rows (stride ldo), one wave per token;
-// the gain comes from field `field` of layer `layer` of the device table, or `gain` when the
-// table is null. out_f32 (optional) receives the bf16 result widened to f32.
-__global__ void __launch_bounds__(256) rmsnorm_kernel(const bf16_t* x, int ldx, const TTSLayerWeights* layers,
-                                                      int layer, int field, const bf16_t* gain, bf16_t* out,
-                                                      int ldo, float* out_f32, int M, int frag) {
-  const int lane = threadIdx.x & 63;
-  const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (m >= M) return;
-  const bf16_t* w = layers ? tbl(layers + layer, field) : gain;
-  const bf16_t* xr = x + (size_t)m * ldx;
-  u32x4 v[2];
   float ss = 0.0f;
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    v[k] = ldw(xr + 8 * (lane + 64 * k));
+  for (int k = 0; k < 2; ++k)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float a = bflo(v[k][e]), b = bfhi(v[k][e]);
-      ss += a * a + b * b;
-    }
-  }
+    for (int e = 0; e < 4; ++e) ss += bflo(v[k][e]) * bflo(v[k][e]) + bfhi(v[k][e]) * bfhi(v[k][e]);
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
   const float rs = 1.0f / sqrtf(ss / (float)HID + EPS);
+  float y[16];
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int e0 = 8 * (lane + 64 * k);
-    const u32x4 gw = ldw(w + e0);
-    u32x4 o;
+  for (int k = 0; k < 2; ++k)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float a = rbf(bflo(gw[e]) * rbf(bflo(v[k][e]) * rs));
-      const float b = rbf(bfhi(gw[e]) * rbf(bfhi(v[k][e]) * rs));
-      o[e] = (uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16);
-      if (out_f32) {
-        out_f32[e0 + 2 * e] = a;
-        out_f32[e0 + 2 * e + 1] = b;
-      }
+      y[8 * k + 2 * e] = rbh(bflo(gw[k][e]) * rbh(bflo(v[k][e]) * rs));
+      y[8 * k + 2 * e + 1] = rbh(bfhi(gw[k][e]) * rbh(bfhi(v[k][e]) * rs));
     }
-    if (out) *reinterpret_cast<u32x4*>(out + (frag ? frag_at(m, e0, ldo) : (size_t)m * ldo + e0)) = o;
+  if (w == 0 && out_hidden != nullptr) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out_hidden[8 * (lane + 64 * k) + e] = y[8 * k + e];
   }
-}
-
-// Per token: q/k head RMSNorm (field 4 / 5 gains), interleaved mRoPE from the bf16 tables, the
-// rotated q written to qdst, the rotated k and the v of every KV head written to the cache at
-// position p0 + s. Lane j of a wave handles channels j and j + 64 (the rotate_half pair). Run by
-// a whole 256-thread workgroup on token s's q | k | v row `src` (global memory or LDS). The table
-// and gain values come first (rope_inputs), so a caller can issue those loads before it builds
-// the row.
-struct RopeIn { float c0, c1, s0, s1, gq0, gq1, gk0, gk1; };
-
-__device__ __forceinline__ RopeIn rope_inputs(int s, const TTSLayerWeights* layers, int layer, const bf16_t* cos_t,
-                                              const bf16_t* sin_t, const int* pos3, int p0, int S, int max_seq) {
-  const int lane = threadIdx.x & 63;
-  const int sec = (lane < 60 && lane % 3 == 1) ? 1 : ((lane < 60 && lane % 3 == 2) ? 2 : 0);
-  // table row of this channel's section (clamped into the table: a caller's out-of-range
-  // position must not read outside it)
-  const int row = pos3 ? min(max(pos3[sec * S + s], 0), max_seq - 1) : p0 + s;
-  const TTSLayerWeights* lw = layers + layer;
-  const bf16_t* qn = tbl(lw, 4);
-  const bf16_t* kn = tbl(lw, 5);
-  RopeIn r;
-  r.c0 = ldbf(cos_t + (size_t)row * HDIM + lane);
-  r.c1 = ldbf(cos_t + (size_t)row * HDIM + lane + 64);
-  r.s0 = ldbf(sin_t + (size_t)row * HDIM + lane);
-  r.s1 = ldbf(sin_t + (size_t)row * HDIM + lane + 64);
-  r.gq0 = ldbf(qn + lane); r.gq1 = ldbf(qn + lane + 64);
-  r.gk0 = ldbf(kn + lane); r.gk1 = ldbf(kn + lane + 64);
-  return r;
-}
-
-__device__ __forceinline__ void rope_kv_apply(const RopeIn& r, const bf16_t* src, bf16_t* qdst, int s, int layer,
-                                              int p0, bf16_t* kc, bf16_t* vc, int max_seq) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int pos = p0 + s;
-  // wave w takes heads w + 4 k (k < 6): q heads for k < 4, k heads 16 + w, 20 + w for k = 4, 5;
-  // every load is issued before the first reduction, the six reductions interleave
-  constexpr int HPW = (NQH + NKVH) / 4;
-  float x0[HPW], x1[HPW], ss[HPW];
+  if (head == nullptr) return;
 #pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const bf16_t* hp = src + (w + 4 * k) * HDIM;
-    x0[k] = bf2f(hp[lane]);
-    x1[k] = bf2f(hp[lane + 64]);
+  for (int r = 0; r < RPW; ++r) {
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += bflo(hw[r][k][e]) * y[8 * k + 2 * e] + bfhi(hw[r][k][e]) * y[8 * k + 2 * e + 1];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0 && RPW * w + r < vocab) logits[RPW * w + r] = f2bh(s);
   }
-#pragma unroll
-  for (int k = 0; k < HPW; ++k) ss[k] = x0[k] * x0[k] + x1[k] * x1[k];
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1)
-#pragma unroll
-    for (int k = 0; k < HPW; ++k) ss[k] += __shfl_xor(ss[k], o, 64);
-#pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const float rs = 1.0f / sqrtf(ss[k] / (float)HDIM + EPS);
-    const float y0 = rbh((k < 4 ? r.gq0 : r.gk0) * rbh(x0[k] * rs));
-    const float y1 = rbh((k < 4 ? r.gq1 : r.gk1) * rbh(x1[k] * rs));
-    const bf16_t o0 = f2bh(rbh(y0 * r.c0) + rbh(-y1 * r.s0));
-    const bf16_t o1 = f2bh(rbh(y1 * r.c1) + rbh(y0 * r.s1));
-    bf16_t* dst = k < 4 ? qdst + (w + 4 * k) * HDIM
-                        : kc + (((size_t)layer * NKVH + (w + 4 * (k - 4))) * max_seq + pos) * HDIM;
-    dst[lane] = o0;
-    dst[lane + 64] = o1;
-  }
-  // v: 8 heads x 128 = 1024 values, 4 per thread
-  const int i0 = 4 * threadIdx.x;
-  const int kvh = i0 >> 7, d = i0 & 127;
-  const u32x2 vv = *reinterpret_cast<const u32x2*>(src + 3072 + i0);
-  *reinterpret_cast<u32x2*>(vc + (((size_t)layer * NKVH + kvh) * max_seq + pos) * HDIM + d) = vv;
-}
-
-__global__ void __launch_bounds__(256) rope_kv_kernel(bf16_t* qkv, const TTSLayerWeights* layers, int layer,
-                                                      const bf16_t* cos_t, const bf16_t* sin_t, const int* pos3,
-                                                      int p0, int S, bf16_t* kc, bf16_t* vc, int max_seq) {
-  const RopeIn r = rope_inputs(blockIdx.x, layers, layer, cos_t, sin_t, pos3, p0, S, max_seq);
-  bf16_t* row = qkv + (size_t)blockIdx.x * QKVW;
-  rope_kv_apply(r, row, row, blockIdx.x, layer, p0, kc, vc, max_seq);   // q rotated in place
-}
-
-// Split-K QKV: token m's 4096 sums in split order -> bf16 q | k | v row in LDS, then the q/k-norm,
-// RoPE and cache write on it, the rotated q to the token's QKV row (one launch instead of a
-// reduction and a rope pass). The table and gain loads go out before the partial sums.
-__global__ void __launch_bounds__(256) reduce_rope_kernel(const GemmArgs g, int splits, const bf16_t* cos_t,
-                                                          const bf16_t* sin_t, const int* pos3, int p0, bf16_t* kc,
-                                                          bf16_t* vc, int max_seq) {
-  __shared__ __attribute__((aligned(16))) bf16_t srow[QKVW];
-  const int m = blockIdx.x;
-  const size_t stride = (size_t)g.M * g.N;
-  const float* P = g.part + (size_t)m * g.N;
-  const RopeIn r = rope_inputs(m, g.layers, g.layer, cos_t, sin_t, pos3, p0, g.M, max_seq);
-  // thread t: elements 16 t .. 16 t + 15, in 16-byte loads
-  const int n0 = 16 * threadIdx.x;
-  float v[16];
-  sum_splits<2, 4>(P + n0, stride, splits, v);
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    u32x4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = pack_bh(v[8 * q + 2 * e], v[8 * q + 2 * e + 1]);
-    *reinterpret_cast<u32x4*>(srow + n0 + 8 * q) = o;
-  }
-  __syncthreads();   // the row is read back by other threads of the workgroup
-  rope_kv_apply(r, srow, g.out + (size_t)m * g.ldo, m, g.layer, p0, kc, vc, max_seq);
-}
-
-// Split-K O or down projection of token m: sums in split order, residual add in place
-// (h = bf16(h + bf16(sum))), then the RMSNorm of the new row with gain field `field` of layer
-// `nlayer` into xn (skipped when nlayer < 0): one launch instead of a reduction and a norm.
-__global__ void __launch_bounds__(256) reduce_resid_norm_kernel(const GemmArgs g, int splits, int nlayer, int field,
-                                                                bf16_t* xn, int frag) {
-  __shared__ float red[4];
-  const int m = blockIdx.x, t = threadIdx.x, lane = t & 63;
-  const size_t stride = (size_t)g.M * g.N;
-  const float* P = g.part + (size_t)m * g.N + 4 * t;
-  bf16_t* hr = g.out + (size_t)m * g.ldo + 4 * t;
-  const u32x2 rv = *reinterpret_cast<const u32x2*>(g.res + (size_t)m * g.ldr + 4 * t);
-  float hv[4];
-  {
-    float sv[4];
-    sum_splits<8, 1>(P, stride, splits, sv);
-    hv[0] = rbh(bflo(rv[0]) + rbh(sv[0]));
-    hv[1] = rbh(bfhi(rv[0]) + rbh(sv[1]));
-    hv[2] = rbh(bflo(rv[1]) + rbh(sv[2]));
-    hv[3] = rbh(bfhi(rv[1]) + rbh(sv[3]));
-  }
-  u32x2 hp;
-  hp[0] = pack_bh(hv[0], hv[1]);
-  hp[1] = pack_bh(hv[2], hv[3]);
-  *reinterpret_cast<u32x2*>(hr) = hp;
-  if (nlayer < 0) return;
-  float ss = hv[0] * hv[0] + hv[1] * hv[1] + hv[2] * hv[2] + hv[3] * hv[3];
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
-  if (lane == 0) red[t >> 6] = ss;
-  __syncthreads();
-  ss = (red[0] + red[1]) + (red[2] + red[3]);
-  const float rs = 1.0f / sqrtf(ss / (float)HID + EPS);
-  const u32x2 gw = *reinterpret_cast<const u32x2*>(tbl(g.layers + nlayer, field) + 4 * t);
-  u32x2 o;
-  o[0] = pack_bh(bflo(gw[0]) * rbh(hv[0] * rs), bfhi(gw[0]) * rbh(hv[1] * rs));
-  o[1] = pack_bh(bflo(gw[1]) * rbh(hv[2] * rs), bfhi(gw[1]) * rbh(hv[3] * rs));
-  *reinterpret_cast<u32x2*>(xn + (frag ? frag_at(m, 4 * t, HID) : (size_t)m * HID + 4 * t)) = o;
 }
 
 // Causal GQA attention of S queries (positions p0 .. p0 + S - 1) over cache positions
@@ -986,9 +166,9 @@ __device__ __forceinline__ u32x2 lds_tr16(const bf16_t* p) {
   return __builtin_bit_cast(u32x2, r);
 }
 
-__global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qkv, const bf16_t* kc, const bf16_t* vc,
+__global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qrows, const bf16_t* kc, const bf16_t* vc,
                                                        int layer, int max_seq, int p0, int S, bf16_t* att,
-                                                       float scale, int frag) {
+                                                       float scale) {
   __shared__ __attribute__((aligned(16))) char smem[ATT_SMEM];
   bf16_t* sq = reinterpret_cast<bf16_t*>(smem);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, hf = lane >> 5, c = lane & 31;
@@ -1009,7 +189,7 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qkv, con
   for (int j = 0; j < 512 / (64 * AW); ++j) {
     const int ch = threadIdx.x + 64 * AW * j, qrow = ch >> 4, qcol = 8 * (ch & 15);
     const int qi = 32 * qb + qrow;
-    const u32x4 v = ldw(qkv + (size_t)(qi < S ? qi : 0) * QKVW + hq * HDIM + qcol);   // clamped row
+    const u32x4 v = ldw(qrows + (size_t)(qi < S ? qi : 0) * (NQH * HDIM) + hq * HDIM + qcol);   // clamped row
     *reinterpret_cast<u32x4*>(&sq[qrow * QROW + qcol]) = qi < S ? v : u32x4{0u, 0u, 0u, 0u};
   }
   __syncthreads();
@@ -1186,8 +366,465 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qkv, con
       u32x2 pk;
       pk[0] = pack_bh(o[mb][4 * rq] * rl, o[mb][4 * rq + 1] * rl);
       pk[1] = pack_bh(o[mb][4 * rq + 2] * rl, o[mb][4 * rq + 3] * rl);
-      *reinterpret_cast<u32x2*>(att + (frag ? frag_at(i, hq * HDIM + d0, NQH * HDIM) : orow + d0)) = pk;
+      *reinterpret_cast<u32x2*>(att + orow + d0) = pk;
     }
+}
+
+// Wait until at most N of this wave's vector-memory instructions are in flight (the compiler does not
+// track LDS writes made by DMA).
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N <= 63, "vmcnt field");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// ... and none of its LDS reads
+template <int N>
+__device__ __forceinline__ void wait_vm_lds() {
+  static_assert(N >= 0 && N <= 63, "vmcnt field");
+  __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+}
+
+// Layer projection C = A W^T of a TM x TN tile (tokens x weight rows), the whole K range in one
+// workgroup, with everything that follows it up to the next matrix product in its epilogue, so that a
+// layer is five launches at every prompt length (QKV, attention, O, gate/up, down):
+//   QKV   rstd, q/k RMSNorm, interleaved mRoPE, K/V cache write (a tile is one head, TN = 128)
+//   GU    rstd, SwiGLU (gate and up rows interleaved by 16)
+//   O, D  residual add, x * gain of the next norm, and the sum of squares that this norm needs
+// RMSNorm is applied around the product: xn = x gain rstd, and rstd is one number per token, so the
+// producer writes bf16(x * gain) with the tile's part of sum(x^2), and the consumer scales its f32 sums by
+// rstd (one bf16 rounding where transformers' form, bf16(gain * bf16(x rstd)), has two). What this removes:
+// split-K partials (f32, written and read back), their reductions and the norms, three launches of 4 to
+// 8 us a layer, each with a launch gap and a memory round trip.
+//
+// Operands are copied global -> LDS by DMA (global_load_lds_dwordx4: each wave instruction writes 64 x 16
+// bytes at a wave-uniform LDS address) through NS stages of BK, NS - 1 of them in flight, one barrier a
+// stage. LDS tile: row r of a stage holds its BK / 8 chunks of 16 bytes with chunk c at position
+// c ^ (r & 7): a DMA instruction reads whole 128- or 256-byte row segments (adjacent lanes on one row: the
+// address unit takes 4 times as long for the MFMA operand order, rows first), and the MFMA operand reads (16
+// rows at one chunk) are conflict-free. Weights are the MFMA's A operand, so a lane ends with 4 consecutive
+// columns of one token: lane l, register e of block (nb, mb) = weight row 16 nb + 4 (l >> 4) + e, token
+// 16 mb + (l & 15). Rows past M read row M - 1; their sums are never stored.
+enum Mode { P_QKV, P_O, P_GU, P_DOWN };
+constexpr int kdim(int mode) { return mode == P_O ? NQH * HDIM : (mode == P_DOWN ? INTER : HID); }
+constexpr int ndim(int mode) { return mode == P_QKV ? 4096 : (mode == P_GU ? 2 * INTER : HID); }
+constexpr int QW = NQH * HDIM;               // a token's rotated queries
+constexpr int SQP = 32;                      // sum-of-squares parts per token (one per column tile)
+
+struct TileArgs {
+  const bf16_t* A;                 // [M, K] activations
+  const TTSLayerWeights* layers;   // device table
+  int layer;
+  int M;
+  int xm, xn;                      // the XCDs as a grid over the tiles: xm x xn = 8
+  const float* ssq;                // QKV, GU: [M][SQP] parts of each token's sum(x^2), nsq of them valid
+  int nsq;
+  bf16_t* out;                     // QKV: q [M, QW]; GU: [M, INTER]
+  bf16_t* h;                       // O, down: residual stream, updated in place
+  bf16_t* xg;                      // ... bf16(h * gain), gain = field nfield of layer nlayer (nlayer < 0: none)
+  float* ssq_out;
+  int nlayer, nfield;
+  const bf16_t* cos_t;             // QKV: tables, (t, h, w) rows [3][M] or nullptr (row = p0 + token), cache
+  const bf16_t* sin_t;
+  const int* pos3;
+  int p0;
+  bf16_t* kc;
+  bf16_t* vc;
+  int max_seq;
+};
+
+// weight row of column n of tile tn (GU: 16 gate rows, then the 16 up rows of the same outputs; FINE, for
+// waves of an odd number of 16-column blocks: 2 gate rows, then the 2 up rows)
+template <int MODE, int TN, bool FINE>
+__device__ __forceinline__ const bf16_t* tile_weight_row(const TTSLayerWeights* lw, int tn, int n) {
+  constexpr int K = kdim(MODE);
+  const int c = tn * TN + n;
+  if constexpr (MODE == P_QKV) {
+    return c < 2048 ? tbl(lw, 1) + (size_t)c * K
+                    : (c < 3072 ? tbl(lw, 2) + (size_t)(c - 2048) * K : tbl(lw, 3) + (size_t)(c - 3072) * K);
+  } else if constexpr (MODE == P_O) {
+    return tbl(lw, 6) + (size_t)c * K;
+  } else if constexpr (MODE == P_GU) {
+    const int row = (TN / 2) * tn + (FINE ? 2 * (n >> 2) + (n & 1) : 16 * (n >> 5) + (n & 15));
+    return ((n >> (FINE ? 1 : 4)) & 1 ? tbl(lw, 9) : tbl(lw, 8)) + (size_t)row * K;
+  } else {
+    return tbl(lw, 10) + (size_t)c * K;
+  }
+}
+
+// q/k RMSNorm and interleaved mRoPE of a tile's head: TM token rows (bf16 rows of pitch tr in LDS, the first
+// one token m0), 8 threads of 8 channel pairs (d, d + 64) a row, to rows of stride ld at dst. The table rows
+// of the next row go out before this one's arithmetic.
+template <int TM, int NT>
+__device__ __forceinline__ void head_finish(const TileArgs& g, const bf16_t* T, int tr, int m0, int t, const bf16_t* gn,
+                                            bf16_t* dst, int ld) {
+  constexpr int RP = NT / 8, NP = (TM + RP - 1) / RP;   // rows a pass, passes
+  const int d0 = 8 * (t & 7);
+  const u32x4 g0 = ldw(gn + d0), g1 = ldw(gn + d0 + 64);
+  auto unpack8 = [](const u32x4& v, float (&f)[8]) QTTS_PF_INLINE {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { f[2 * e] = bflo(v[e]); f[2 * e + 1] = bfhi(v[e]); }
+  };
+  struct Cs { u32x4 c0, c1, s0, s1; };
+  auto load = [&](int row) QTTS_PF_INLINE {
+    const int m = min(m0 + min(row, TM - 1), g.M - 1);
+    Cs r;
+    if (g.pos3 == nullptr) {
+      const size_t ro = (size_t)(g.p0 + m) * HDIM + d0;
+      r = {ldw(g.cos_t + ro), ldw(g.cos_t + ro + 64), ldw(g.sin_t + ro), ldw(g.sin_t + ro + 64)};
+    } else {
+      // table rows of the three sections (t, h, w); channel d < 60 takes h when d % 3 == 1 and w when
+      // d % 3 == 2, every other channel t (the same row for d and d + 64); clamped into the table
+      Cs v[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const size_t ro = (size_t)min(max(g.pos3[j * g.M + m], 0), g.max_seq - 1) * HDIM + d0;
+        v[j] = {ldw(g.cos_t + ro), ldw(g.cos_t + ro + 64), ldw(g.sin_t + ro), ldw(g.sin_t + ro + 64)};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        auto sec = [&](int k) QTTS_PF_INLINE { const int d = d0 + k; return d < 60 ? d % 3 : 0; };
+        const int a = sec(2 * e), b = sec(2 * e + 1);
+        auto pick = [&](uint32_t x, uint32_t y, uint32_t z) QTTS_PF_INLINE {
+          const uint32_t lo = a == 0 ? x : (a == 1 ? y : z), hi = b == 0 ? x : (b == 1 ? y : z);
+          return (lo & 0xffffu) | (hi & 0xffff0000u);
+        };
+        r.c0[e] = pick(v[0].c0[e], v[1].c0[e], v[2].c0[e]);
+        r.c1[e] = pick(v[0].c1[e], v[1].c1[e], v[2].c1[e]);
+        r.s0[e] = pick(v[0].s0[e], v[1].s0[e], v[2].s0[e]);
+        r.s1[e] = pick(v[0].s1[e], v[1].s1[e], v[2].s1[e]);
+      }
+    }
+    return r;
+  };
+  Cs cs[2];
+  cs[0] = load(t >> 3);
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int row = (t >> 3) + RP * p;
+    if (p + 1 < NP) cs[(p + 1) & 1] = load(row + RP);
+    if (TM < RP && row >= TM) break;
+    const u32x4 xa = *reinterpret_cast<const u32x4*>(T + row * tr + d0);
+    const u32x4 xb = *reinterpret_cast<const u32x4*>(T + row * tr + d0 + 64);
+    float x0[8], x1[8], c0[8], c1[8], s0[8], s1[8], ga[8], gb[8];
+    unpack8(xa, x0); unpack8(xb, x1);
+    const Cs& c = cs[p & 1];
+    unpack8(c.c0, c0); unpack8(c.c1, c1); unpack8(c.s0, s0); unpack8(c.s1, s1); unpack8(g0, ga); unpack8(g1, gb);
+    float ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ss += x0[k] * x0[k] + x1[k] * x1[k];
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    const float rs = 1.0f / sqrtf(ss / (float)HDIM + EPS);
+    float r0[8], r1[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float y0 = rbh(ga[k] * rbh(x0[k] * rs)), y1 = rbh(gb[k] * rbh(x1[k] * rs));
+      r0[k] = rbh(y0 * c0[k]) + rbh(-y1 * s0[k]);
+      r1[k] = rbh(y1 * c1[k]) + rbh(y0 * s1[k]);
+    }
+    u32x4 o0, o1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o0[e] = pack_bh(r0[2 * e], r0[2 * e + 1]);
+      o1[e] = pack_bh(r1[2 * e], r1[2 * e + 1]);
+    }
+    if (m0 + row < g.M) {
+      *reinterpret_cast<u32x4*>(dst + (size_t)row * ld + d0) = o0;
+      *reinterpret_cast<u32x4*>(dst + (size_t)row * ld + d0 + 64) = o1;
+    }
+  }
+}
+
+template <int MODE, int TM, int TN, int NWM, int NWN, int NWK, int NS, int BK>
+__global__ void __launch_bounds__(64 * NWM * NWN * NWK, 2) tile_gemm_kernel(const TileArgs g) {
+  constexpr int K = kdim(MODE), NW = NWM * NWN * NWK, NT = 64 * NW, NK = K / BK;
+  constexpr int KK = BK / 32 / NWK;                         // a wave's MFMA steps per stage
+  constexpr int CPR = BK / 8, RPI = 64 / CPR;               // 16-byte chunks per row, rows per DMA instruction
+  constexpr int NIW = (TM + TN) / RPI / NW;                 // DMA instructions per wave and stage
+  constexpr int STAGE = (TM + TN) * BK * 2;
+  constexpr int MB = TM / NWM / 16, NB = TN / NWN / 16;     // a wave's 16 x 16 blocks
+  constexpr bool NORMED = MODE == P_QKV || MODE == P_GU;
+  constexpr int TR = HDIM + 8;                              // QKV: bf16 row of the staged head tile
+  static_assert((TM + TN) % (RPI * NW) == 0 && TM % RPI == 0 && K % BK == 0 && NK >= NS - 1, "stages");
+  static_assert(KK >= 2 && KK % 2 == 0 && NWK * NWM * NWN == NW, "operand double buffer");
+  static_assert(NWK == 1 || (NWK - 1) * TM * TN * 4 <= NS * STAGE, "K parts of the sums");
+  static_assert(MODE != P_QKV || (TN == HDIM && TM * TR * 2 <= NS * STAGE), "QKV: one head per tile");
+  constexpr bool FINE = MODE == P_GU && (TN / NWN) % 32 != 0;   // gate/up interleave (tile_weight_row)
+  static_assert(ndim(MODE) % TN == 0 && (MODE == P_QKV || MODE == P_GU || ndim(MODE) / TN <= SQP), "column tiles");
+  // one LDS object: with several, the compiler tracks which of them a DMA may write and waits for every
+  // DMA in flight before each LDS read
+  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE + (NORMED ? 1 : NWN) * TM * 4];
+  float* rstd = reinterpret_cast<float*>(lds + NS * STAGE);   // NORMED
+  float* sred = rstd;                                         // O, down: the waves' sums of squares
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = w % NWM, wn = w / NWM % NWN, wk = w / (NWM * NWN);
+  // XCD-aware tile order: workgroups reach the XCDs round-robin by linear id; XCD x takes the sub-grid
+  // (x % xm, x / xm) of the tiles, row tiles first
+  const int tm_n = (g.M + TM - 1) / TM, x = blockIdx.x & 7, r0 = blockIdx.x >> 3;
+  const int mx = tm_n / g.xm, nx = ndim(MODE) / TN / g.xn;
+  const int tm = (x % g.xm) * mx + r0 % mx, tn = (x / g.xm) * nx + r0 / mx;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const TTSLayerWeights* lw = g.layers + g.layer;
+
+  // loads that the epilogue needs go out ahead of the DMA: the row's sum-of-squares parts, or the residual
+  // and the next norm's gain
+  const int lm = 16 * MB * wm + (lane & 15), ln = 16 * NB * wn + 4 * (lane >> 4);   // this lane's first token, column
+  float sq[NORMED ? (TM + NT - 1) / NT : 1];
+  u32x2 hr[NORMED ? 1 : MB][NORMED ? 1 : NB], gw[NORMED ? 1 : NB];
+  if constexpr (NORMED) {
+#pragma unroll
+    for (int i = 0; i < (TM + NT - 1) / NT; ++i) {
+      const int m = min(m0 + t + NT * i, g.M - 1);
+      float s = 0.0f;
+      const u32x4* p = reinterpret_cast<const u32x4*>(g.ssq + (size_t)m * SQP);
+#pragma unroll
+      for (int q = 0; q < SQP / 4; ++q) {
+        const u32x4 v = p[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += 4 * q + e < g.nsq ? __uint_as_float(v[e]) : 0.0f;
+      }
+      sq[i] = s;
+    }
+  } else {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        hr[mb][nb] = *reinterpret_cast<const u32x2*>(g.h + (size_t)min(m0 + lm + 16 * mb, g.M - 1) * HID + n0 + ln + 16 * nb);
+    const bf16_t* gp = tbl(g.layers + max(g.nlayer, 0), g.nfield);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) gw[nb] = *reinterpret_cast<const u32x2*>(gp + n0 + ln + 16 * nb);
+  }
+
+  // this lane's source of DMA instruction i: stage row RPI (NIW w + i) + lane / CPR (token rows, then
+  // weight rows), the chunk that belongs at position lane % CPR
+  const bf16_t* src[NIW];
+#pragma unroll
+  for (int i = 0; i < NIW; ++i) {
+    const int r = RPI * (NIW * w + i) + lane / CPR, c = (lane % CPR) ^ (r & 7);
+    const bf16_t* p = r < TM ? g.A + (size_t)min(m0 + r, g.M - 1) * K : tile_weight_row<MODE, TN, FINE>(lw, tn, r - TM);
+    src[i] = p + 8 * c;
+  }
+  auto issue = [&](int s, int kt) QTTS_PF_INLINE {   // stage s <- K step kt (clamped: past the end the last one again)
+    const int k = BK * min(kt, NK - 1);
+    char* base = lds + s * STAGE + 1024 * NIW * w;
+#pragma unroll
+    for (int i = 0; i < NIW; ++i)
+      __builtin_amdgcn_global_load_lds((gvoid_t*)(src[i] + k), (lvoid_t*)(base + 1024 * i), 16, 0, 0);
+  };
+  f32x4 acc[NB][MB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // MFMA operands of step i of stage s: (stage row r, chunk c) at byte r BK 2 + 16 (c ^ (r & 7)); r & 7 is
+  // the lane's alone (block rows are multiples of 16)
+  bf16x8 av[2][MB], bv[2][NB];
+  auto read = [&](int s, int i, bf16x8 (&x)[MB], bf16x8 (&y)[NB]) QTTS_PF_INLINE {
+    const int co = ((4 * (i * NWK + wk) + (lane >> 4)) ^ (lane & 7)) * 16;
+    const char* a = lds + s * STAGE + (16 * MB * wm + (lane & 15)) * BK * 2 + co;
+    const char* b = lds + s * STAGE + (TM + 16 * NB * wn + (lane & 15)) * BK * 2 + co;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) y[nb] = as_bf8(*reinterpret_cast<const u32x4*>(b + nb * 16 * BK * 2));
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) x[mb] = as_bf8(*reinterpret_cast<const u32x4*>(a + mb * 16 * BK * 2));
+  };
+  auto mfma = [&](const bf16x8 (&x)[MB], const bf16x8 (&y)[NB]) QTTS_PF_INLINE {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        acc[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y[nb], x[mb], acc[nb][mb], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(s, s);
+  if constexpr (NORMED) {
+#pragma unroll
+    for (int i = 0; i < (TM + NT - 1) / NT; ++i)
+      if (t + NT * i < TM) rstd[t + NT * i] = 1.0f / sqrtf(sq[i] / (float)HID + EPS);
+  }
+  // The operands of each step are read one step ahead, those of a stage's first step before the last MFMAs
+  // of the stage before it, so that the LDS reads run under the MFMAs.
+  // Next stage kt: this wave's DMA has landed and its reads of the stage before are done; then every
+  // wave's, and the buffer of the stage before is free for stage kt + NS - 1.
+  auto next = [&](int kt, int free_buf) QTTS_PF_INLINE {
+    wait_vm_lds<(NS - 2) * NIW>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");   // no LDS access moves across
+    issue(free_buf, kt + NS - 1);
+  };
+  next(0, NS - 1);
+  read(0, 0, av[0], bv[0]);
+  int st = 0;
+#pragma unroll 1
+  for (int kt = 0; kt < NK; ++kt) {
+    const int sn = st + 1 == NS ? 0 : st + 1;
+#pragma unroll
+    for (int i = 0; i < KK; ++i) {
+      if (i + 1 < KK) {
+        read(st, i + 1, av[(i + 1) & 1], bv[(i + 1) & 1]);
+      } else {
+        next(kt + 1, st);            // (past the last stage: clamped copies that nothing uses)
+        read(sn, 0, av[0], bv[0]);
+      }
+      mfma(av[i & 1], bv[i & 1]);
+    }
+    st = sn;
+  }
+  wait_vm_lds<0>();                  // no DMA may still target LDS when it is used again or given back
+  __syncthreads();
+  if constexpr (NWK > 1) {
+    // the waves of a tile part add their K parts, in K order
+    float* part = reinterpret_cast<float*>(lds);
+    constexpr int PW = NWM * NWN * NB * MB * 4 * 64;   // floats of one K part
+    const int at = (wm + NWM * wn) * NB * MB * 4 * 64 + lane * 4;
+    if (wk > 0) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          *reinterpret_cast<f32x4*>(part + (wk - 1) * PW + at + (nb * MB + mb) * 256) = acc[nb][mb];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int j = 0; j < NWK - 1; ++j)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) acc[nb][mb] += *reinterpret_cast<const f32x4*>(part + j * PW + at + (nb * MB + mb) * 256);
+    }
+    if constexpr (MODE == P_QKV) __syncthreads();     // the parts have been read: their LDS takes the head tile
+  }
+
+  if constexpr (MODE == P_QKV) {
+    bf16_t* T = reinterpret_cast<bf16_t*>(lds);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      if (wk > 0) break;
+      const float rs = rstd[lm + 16 * mb];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const f32x4 v = acc[nb][mb];
+        u32x2 o;
+        o[0] = pack_bh(v[0] * rs, v[1] * rs);
+        o[1] = pack_bh(v[2] * rs, v[3] * rs);
+        *reinterpret_cast<u32x2*>(T + (lm + 16 * mb) * TR + ln + 16 * nb) = o;
+      }
+    }
+    __syncthreads();
+    const int head = tn;   // q heads 0..15, k heads 16..23, v heads 24..31
+    if (head >= NQH + NKVH) {
+      bf16_t* vbase = g.vc + ((size_t)g.layer * NKVH + (head - NQH - NKVH)) * g.max_seq * HDIM;
+      for (int q = t; q < TM * 16; q += NT) {
+        const int row = q >> 4, ch = 8 * (q & 15), m = m0 + row;
+        if (m < g.M)
+          *reinterpret_cast<u32x4*>(vbase + (size_t)(g.p0 + m) * HDIM + ch) = *reinterpret_cast<const u32x4*>(T + row * TR + ch);
+      }
+      return;
+    }
+    const bool isq = head < NQH;
+    const bf16_t* gn = tbl(lw, isq ? 4 : 5);
+    head_finish<TM, NT>(g, T, TR, m0, t, gn,
+                        isq ? g.out + (size_t)m0 * QW + head * HDIM
+                            : g.kc + (((size_t)g.layer * NKVH + (head - NQH)) * g.max_seq + g.p0 + m0) * HDIM,
+                        isq ? QW : HDIM);
+  } else if constexpr (MODE == P_GU) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = m0 + lm + 16 * mb;
+      const float rs = rstd[lm + 16 * mb];
+      if (m >= g.M || wk > 0) continue;
+      bf16_t* o = g.out + (size_t)m * INTER + n0 / 2 + 8 * NB * wn + 4 * (lane >> 4);
+      if constexpr (FINE) {
+        // (gate, gate, up, up) of outputs 8 nb + 2 (l >> 4) + {0, 1}
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const f32x4 v = acc[nb][mb];
+          const float a0 = rbh(silu_f(rbh(v[0] * rs))) * rbh(v[2] * rs), a1 = rbh(silu_f(rbh(v[1] * rs))) * rbh(v[3] * rs);
+          *reinterpret_cast<uint32_t*>(o - 2 * (lane >> 4) + 8 * nb) = pack_bh(a0, a1);
+        }
+        continue;
+      }
+#pragma unroll
+      for (int p = 0; p < NB / 2; ++p) {
+        const f32x4 gs = acc[2 * p][mb], us = acc[2 * p + 1][mb];
+        float a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = rbh(silu_f(rbh(gs[e] * rs))) * rbh(us[e] * rs);
+        u32x2 v;
+        v[0] = pack_bh(a[0], a[1]);
+        v[1] = pack_bh(a[2], a[3]);
+        *reinterpret_cast<u32x2*>(o + 16 * p) = v;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      if (wk > 0) break;
+      const int m = m0 + lm + 16 * mb;
+      float ss = 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const f32x4 v = acc[nb][mb];
+        const u32x2 r = hr[mb][nb];
+        const float a0 = rbh(bflo(r[0]) + rbh(v[0])), a1 = rbh(bfhi(r[0]) + rbh(v[1]));
+        const float a2 = rbh(bflo(r[1]) + rbh(v[2])), a3 = rbh(bfhi(r[1]) + rbh(v[3]));
+        ss += (a0 * a0 + a1 * a1) + (a2 * a2 + a3 * a3);
+        if (m < g.M) {
+          const size_t at = (size_t)m * HID + n0 + ln + 16 * nb;
+          u32x2 o;
+          o[0] = pack_bh(a0, a1);
+          o[1] = pack_bh(a2, a3);
+          *reinterpret_cast<u32x2*>(g.h + at) = o;
+          if (g.nlayer >= 0) {
+            u32x2 y;
+            y[0] = pack_bh(a0 * bflo(gw[nb][0]), a1 * bfhi(gw[nb][0]));
+            y[1] = pack_bh(a2 * bflo(gw[nb][1]), a3 * bfhi(gw[nb][1]));
+            *reinterpret_cast<u32x2*>(g.xg + at) = y;
+          }
+        }
+      }
+      ss += __shfl_xor(ss, 16, 64);
+      ss += __shfl_xor(ss, 32, 64);
+      if (lane < 16) sred[wn * TM + lm + 16 * mb] = ss;
+    }
+    __syncthreads();
+    for (int q = t; q < TM; q += NT) {
+      float s = sred[q];
+#pragma unroll
+      for (int j = 1; j < NWN; ++j) s += sred[j * TM + q];
+      if (m0 + q < g.M) g.ssq_out[(size_t)(m0 + q) * SQP + tn] = s;
+    }
+  }
+}
+
+// The prompt embeddings into the residual stream, with bf16(x * gain) and sum(x^2) of layer 0's input
+// norm; one wave per token.
+__global__ void __launch_bounds__(256) embed_kernel(const bf16_t* x, const TTSLayerWeights* layers, bf16_t* h, bf16_t* xg,
+                                                    float* ssq, int M) {
+  const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= M) return;
+  const bf16_t* w = tbl(layers, 0);
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int e0 = 8 * (lane + 64 * k);
+    const u32x4 v = ldw(x + (size_t)m * HID + e0), gw = ldw(w + e0);
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = bflo(v[e]), b = bfhi(v[e]);
+      ss += a * a + b * b;
+      o[e] = pack_bh(a * bflo(gw[e]), b * bfhi(gw[e]));
+    }
+    *reinterpret_cast<u32x4*>(h + (size_t)m * HID + e0) = v;
+    *reinterpret_cast<u32x4*>(xg + (size_t)m * HID + e0) = o;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  if (lane == 0) ssq[(size_t)m * SQP] = ss;
 }
 
 // First group-0 token from bf16 logits: ids [n-1024, n) except EOS suppressed when mask_tail
@@ -1196,68 +833,88 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qkv, con
 __global__ void __launch_bounds__(64) select_kernel(const bf16_t* logits, int n, int mask_tail, int eos_id,
                                                     int suppress_eos, SelParams sp, float* out_logits,
                                                     int* out_token) {
-  __shared__ float stage[MAXV];
   __shared__ SelScratch sc;
   const int lane = threadIdx.x;
   // every logit load is issued before the first is used (a rolled loop waited for each in turn);
   // loads past n are clamped to n - 1 and dropped
-  constexpr int NJ = (MAXV + 63) / 64;
-  float lv[NJ];
+  bf16_t lv[SEL_NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) lv[j] = bf2f(logits[min(lane + 64 * j, n - 1)]);
+  for (int j = 0; j < SEL_NJ; ++j) lv[j] = *gmem(logits + min(lane + 64 * j, n - 1));
+  uint32_t w[SEL_NJ], best = 0u;
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
+  for (int j = 0; j < SEL_NJ; ++j) {
     const int i = lane + 64 * j;
-    if (i >= n) break;
-    float v = lv[j];
-    if (out_logits) out_logits[i] = v;
-    if (mask_tail && i >= n - 1024 && i != eos_id) v = -INFINITY;
-    if (suppress_eos && i == eos_id) v = -INFINITY;
-    stage[i] = v;
+    float v = bf2f(lv[j]);
+    if (out_logits && i < n) out_logits[i] = v;
+    if ((mask_tail && i >= n - 1024 && i != eos_id) || (suppress_eos && i == eos_id)) v = -INFINITY;
+    w[j] = i < n ? (bfkey(v) << 16) | (uint32_t)i : 0u;
+    best = max(best, i < n ? greedy_word(v, i) : 0u);
   }
-  __syncthreads();
-  const int tok = wave_select(stage, n, sp, &sc);
+  const int tok = sp.do_sample ? wave_sample(w, n, sp, &sc) : greedy_id(best, n);
   if (lane == 0) *out_token = tok;
 }
 
 // ---- host ----------------------------------------------------------------------------------
 
-struct Shape { int N, K; };
-constexpr Shape kQKV{4096, HID}, kO{HID, NQH * HDIM}, kGU{2 * INTER, HID}, kDown{HID, INTER};
-
-// tile width: 128 columns from 256 rows on (one LDS read per MFMA), 64 below (more tiles for
-// the weight-streaming small-M case)
-int tile_n(int M) { return M >= 256 ? 128 : 64; }
-
-// split-K factor: double while the tile grid is below its target and the K range still splits
-// into whole K steps. Targets: 128 workgroups below 256 rows (every split writes a full f32
-// partial tile, which at 128 rows outweighs the weights it streams), one per CU from 256 rows.
-// The SwiGLU GEMM is never split: its fused epilogue beats the unfused reduction at every M
-// (measured at 128, 512 and 2048 rows), and its tile grid is the widest of the layer.
-int splits_for(int M, int N, int K, bool swiglu = false) {
-  if (swiglu) return 1;
-  const int tn = tile_n(M), bk = tn == 64 ? bk_of<64>() : bk_of<128>();
-  const int tiles = ((M + BM - 1) / BM) * (N / tn);
-  const int target = M >= 256 ? 256 : 128;
-  int ks = 1;
-  while (tiles * ks < target && ks < MAX_SPLIT && (K / bk) % (2 * ks) == 0) ks *= 2;
-  return ks;
+// One launch of a projection: tile TM x TN (NWM x NWN waves), NS stages of BK.
+template <int MODE, int TM, int TN, int NWM, int NWN, int NWK, int NS, int BK>
+void launch_tile(TileArgs& g, hipStream_t st) {
+  const int tm = (g.M + TM - 1) / TM, tn = ndim(MODE) / TN;
+  // the XCD grid xm x xn that re-reads least: every XCD column reads the activations, every XCD row the weights
+  g.xm = 1;
+  double best = 1e30;
+  for (int xm = 1; xm <= 8; xm *= 2) {
+    if (tm % xm != 0 || tn % (8 / xm) != 0) continue;
+    const double cost = (double)g.M * (8 / xm) + (double)ndim(MODE) * xm;
+    if (cost < best) { best = cost; g.xm = xm; }
+  }
+  g.xn = 8 / g.xm;
+  static_assert(ndim(MODE) / TN % 8 == 0, "column tiles over the XCDs");
+  hipLaunchKernelGGL((tile_gemm_kernel<MODE, TM, TN, NWM, NWN, NWK, NS, BK>), dim3(tm * tn), dim3(64 * NWM * NWN * NWK), 0, st, g);
 }
 
-// The row GEMM (M <= RM) per projection: tile width and split count, for a grid of 192-256
-// workgroups (QKV 128 tiles x 2 splits, O and down 32 tiles x 8, gate/up 192 tiles unsplit)
-constexpr int rows_tn(int) { return 32; }
-constexpr int rows_ks(int wm) { return wm == W_QKV ? 2 : (wm == W_GU ? 1 : 8); }
-constexpr Shape shape_of(int wm) { return wm == W_QKV ? kQKV : (wm == W_O ? kO : (wm == W_GU ? kGU : kDown)); }
-int splits_of(int wm, int M) {
-  const Shape sh = shape_of(wm);
-  return M <= RM ? rows_ks(wm) : splits_for(M, sh.N, sh.K, wm == W_GU);
+// Tiles by prompt length M. A projection's time is its workgroups' K loop (operand bytes per CU through
+// LDS) plus about 4 us of launch, first loads and epilogue, so the tile grows with M as slowly as 256
+// workgroups, one a CU, allow. Measured over prompts of 13 to 2048 tokens (us a layer, against the best
+// alternative):
+//   QKV (a head's 128 columns)  32 tokens up to 256, 64 to 512, 128 to 1024, then 256; a step too small
+//                               or too large costs 2 to 10 us
+//   GU    16 x 64 up to 32 tokens (at 13: 1.2 us less than 32 x 96), 32 x 96 to 128, 64 x 96 to 256 (32 x 96:
+//         +1.8 to 2.1), 64 x 192 to 512 (64 x 96: +1.4 to 2.1), 128 x 192 to 1024, then 256 x 192 (at 1500:
+//         3.9 less)
+//   O, D  16 x 32 up to 128, 32 x 32 to 256 (+2 to 3 either way), 32 x 64 to 512, 64 x 64 to 1024, then
+//         128 x 64; two or four waves share a block's K range where one wave's chain of MFMAs and LDS reads
+//         is what a stage waits for (0.7 to 2 us less each)
+void project_qkv(TileArgs& g, hipStream_t st) {
+  if (g.M <= 256) launch_tile<P_QKV, 32, 128, 1, 4, 1, 6, 64>(g, st);
+  else if (g.M <= 512) launch_tile<P_QKV, 64, 128, 2, 2, 1, 5, 64>(g, st);
+  else if (g.M <= 1024) launch_tile<P_QKV, 128, 128, 4, 2, 1, 4, 64>(g, st);
+  else launch_tile<P_QKV, 256, 128, 4, 2, 1, 3, 64>(g, st);
 }
+void project_gate_up(TileArgs& g, hipStream_t st) {
+  if (g.M <= 32) launch_tile<P_GU, 16, 64, 1, 4, 1, 4, 128>(g, st);
+  else if (g.M <= 128) launch_tile<P_GU, 32, 96, 2, 2, 1, 4, 64>(g, st);
+  else if (g.M <= 256) launch_tile<P_GU, 64, 96, 2, 2, 1, 3, 64>(g, st);
+  else if (g.M <= 512) launch_tile<P_GU, 64, 192, 2, 2, 1, 4, 64>(g, st);
+  else if (g.M <= 1024) launch_tile<P_GU, 128, 192, 4, 2, 1, 3, 64>(g, st);
+  else launch_tile<P_GU, 256, 192, 4, 2, 1, 2, 64>(g, st);
+}
+// O or down: also leaves in g.nsq how many sum-of-squares parts it wrote per token
+template <int MODE>
+void project_residual(TileArgs& g, hipStream_t st) {
+  g.nsq = g.M <= 256 ? HID / 32 : HID / 64;
+  if (g.M <= 128) launch_tile<MODE, 16, 32, 1, 2, 4, 5, 256>(g, st);
+  else if (g.M <= 256) launch_tile<MODE, 32, 32, 2, 2, 2, 6, 128>(g, st);
+  else if (g.M <= 512) launch_tile<MODE, 32, 64, 2, 2, 2, 5, 128>(g, st);
+  else if (g.M <= 1024) launch_tile<MODE, 64, 64, 2, 2, 2, 4, 128>(g, st);
+  else launch_tile<MODE, 128, 64, 2, 2, 2, 3, 128>(g, st);
+}
+
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct Layout {
-  size_t h, xn, qkv, att, act, hb, logits, part, total;
+  size_t h, xg, ssq, q, att, act, logits, total;
 };
 
 Layout layout(int S, int vocab) {
@@ -1265,73 +922,14 @@ Layout layout(int S, int vocab) {
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o = align256(o + bytes); return at; };
   L.h = take((size_t)S * HID * 2);
-  // the row GEMM's token operands hold whole 16-row blocks
-  const size_t SP = S <= RM ? (size_t)(S + 15) / 16 * 16 : (size_t)S;
-  L.xn = take(SP * HID * 2);
-  L.qkv = take((size_t)S * QKVW * 2);
-  L.att = take(SP * NQH * HDIM * 2);
-  L.act = take(SP * INTER * 2);
-  L.hb = take(HID * 2);
+  L.xg = take((size_t)S * HID * 2);
+  L.ssq = take((size_t)S * SQP * 4);
+  L.q = take((size_t)S * QW * 2);
+  L.att = take((size_t)S * QW * 2);
+  L.act = take((size_t)S * INTER * 2);
   L.logits = take((size_t)(vocab > 0 ? vocab : MAXV) * 2);
-  size_t pb = 0;
-  for (int wm : {W_QKV, W_O, W_DOWN}) {
-    const int ks = splits_of(wm, S);
-    if (ks > 1) pb = std::max(pb, (size_t)ks * S * shape_of(wm).N * 4);
-  }
-  const int ksh = splits_for(1, vocab > 0 ? vocab : MAXV, HID);
-  if (ksh > 1) pb = std::max(pb, (size_t)ksh * (vocab > 0 ? vocab : MAXV) * 4);
-  L.part = take(pb);
   L.total = o;
   return L;
-}
-
-template <int WM, int EPI, int TN>
-void gemm_launch(const GemmArgs& g, int ks, bool reduce, hipStream_t st) {
-  dim3 grid(g.N / TN, (g.M + BM - 1) / BM, ks);
-  hipLaunchKernelGGL((gemm_kernel<WM, EPI, TN>), grid, dim3(GT), 0, st, g);
-  if (ks > 1 && reduce) {
-    const long nout = (long)g.M * (EPI == E_SWIGLU ? g.N / 2 : g.N) / 4;
-    hipLaunchKernelGGL((reduce_kernel<EPI, TN>), dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, st, g, ks);
-  }
-}
-
-// Launches the GEMM; with split-K the partial sums are left in g.part for a fused consumer when
-// `reduce` is false, else reduced here. `rope` (QKV only): an unsplit 128-column QKV GEMM finishes
-// the heads itself (q/k-norm, RoPE, K/V write). Returns the split count (0 on a launch error).
-template <int WM, int EPI>
-int gemm(GemmArgs& g, hipStream_t st, bool reduce = true, const RopeArgs* rope = nullptr) {
-  if constexpr (WM != W_DIRECT) {
-    if (g.M <= RM) {
-      constexpr int TN = rows_tn(WM), KS = rows_ks(WM), K = shape_of(WM).K;
-      static_assert(K % (KS * 128) == 0 && (KS == 1 || EPI != E_SWIGLU), "row GEMM plan");
-      if (g.K != K || g.N != shape_of(WM).N) return 0;
-      g.kchunk = K / KS;
-      hipLaunchKernelGGL((gemm_rows_kernel<WM, EPI, TN, K / KS / 128>), dim3(g.N / TN, 1, KS), dim3(GT), 0, st, g);
-      if (KS > 1 && reduce)
-        hipLaunchKernelGGL((reduce_kernel<EPI, 64>), dim3((unsigned)(((long)g.M * g.N / 4 + 255) / 256)), dim3(256), 0,
-                           st, g, KS);
-      return hipGetLastError() == hipSuccess ? KS : 0;
-    }
-  }
-  const int ks = splits_for(g.M, g.N, g.K, EPI == E_SWIGLU);
-  g.kchunk = g.K / ks;
-  if (tile_n(g.M) == 128) {
-    // two stages and two workgroups per CU when the grid covers the CUs twice or more; a grid of
-    // at most one workgroup per CU (the split O and down projections) takes three stages instead
-    const dim3 grid(g.N / 128, (g.M + 127) / 128, ks);
-    const RopeArgs rr = (rope != nullptr && ks == 1) ? *rope : RopeArgs{};
-    if (grid.x * grid.y * grid.z > 256)
-      hipLaunchKernelGGL((gemm_dma_kernel<WM, EPI, 2>), grid, dim3(GT), 0, st, g, rr);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<WM, EPI, 3>), grid, dim3(GT), 0, st, g, rr);
-    if (ks > 1 && reduce) {
-      const long nout = (long)g.M * (EPI == E_SWIGLU ? g.N / 2 : g.N) / 4;
-      hipLaunchKernelGGL((reduce_kernel<EPI, 128>), dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, st, g, ks);
-    }
-  } else {
-    gemm_launch<WM, EPI, 64>(g, ks, reduce, st);
-  }
-  return hipGetLastError() == hipSuccess ? ks : 0;
 }
 
 }  // namespace pf
@@ -1368,79 +966,54 @@ hipError_t qtts_backbone_prefill(void* workspace, size_t workspace_bytes, const 
   if (workspace_bytes < L.total) return hipErrorInvalidValue;
   char* ws = static_cast<char*>(workspace);
   bf16_t* h = reinterpret_cast<bf16_t*>(ws + L.h);
-  bf16_t* xn = reinterpret_cast<bf16_t*>(ws + L.xn);
-  bf16_t* qkv = reinterpret_cast<bf16_t*>(ws + L.qkv);
+  bf16_t* xg = reinterpret_cast<bf16_t*>(ws + L.xg);
+  float* ssq = reinterpret_cast<float*>(ws + L.ssq);
+  bf16_t* q = reinterpret_cast<bf16_t*>(ws + L.q);
   bf16_t* att = reinterpret_cast<bf16_t*>(ws + L.att);
   bf16_t* act = reinterpret_cast<bf16_t*>(ws + L.act);
-  bf16_t* hb = reinterpret_cast<bf16_t*>(ws + L.hb);
-  float* part = reinterpret_cast<float*>(ws + L.part);
   auto* kc = static_cast<bf16_t*>(k_cache);
   auto* vc = static_cast<bf16_t*>(v_cache);
   const auto* cs = static_cast<const bf16_t*>(cos_table);
   const auto* sn = static_cast<const bf16_t*>(sin_table);
   const float scale = 1.0f / sqrtf((float)HDIM);
   const unsigned norm_grid = (unsigned)((S + 3) / 4);
-  // prompts the row GEMM takes: its token operands (xn, att, act) in the token-fragment layout
-  const int frag = S <= RM ? 1 : 0;
-
-  hipError_t e = hipMemcpyAsync(h, input_embeddings, (size_t)S * HID * 2, hipMemcpyDeviceToDevice, stream);
-  if (e != hipSuccess) return e;
-  // layer 0's input norm; later input norms come with the previous layer's down projection
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(norm_grid), dim3(256), 0, stream, h, HID, layer_weights, 0, 0,
-                     (const bf16_t*)nullptr, xn, HID, (float*)nullptr, S, frag);
-  const unsigned rows = (unsigned)S;
-  const RopeArgs rope{cs, sn, pos3, position, kc, vc, max_seq_len};
+  hipLaunchKernelGGL(embed_kernel, dim3(norm_grid), dim3(256), 0, stream, static_cast<const bf16_t*>(input_embeddings),
+                     layer_weights, h, xg, ssq, S);
+  TileArgs g{};
+  g.layers = layer_weights;
+  g.M = S;
+  g.ssq = ssq;
+  g.ssq_out = ssq;
+  g.h = h;
+  g.xg = xg;
+  g.cos_t = cs;
+  g.sin_t = sn;
+  g.pos3 = pos3;
+  g.p0 = position;
+  g.kc = kc;
+  g.vc = vc;
+  g.max_seq = max_seq_len;
+  g.nsq = 1;   // the embeddings' sums of squares are whole
   for (int l = 0; l < num_layers; ++l) {
-    GemmArgs g{};
-    g.layers = layer_weights;
     g.layer = l;
-    g.M = S;
-    g.part = part;
-    int ks;
-    // QKV, then q/k-norm + RoPE + K/V write: in the GEMM's epilogue (unsplit 128-column tiles), in
-    // the split-K reduction, or (64-column tiles, unsplit) in rope_kv_kernel
-    g.A = xn; g.lda = HID; g.N = kQKV.N; g.K = kQKV.K; g.out = qkv; g.ldo = QKVW;
-    if ((ks = gemm<W_QKV, E_STORE>(g, stream, false, &rope)) == 0) return hipGetLastError();
-    if (ks == 1 && tile_n(S) == 128) {
-      // q/k-norm, RoPE and the K/V write ran in the QKV GEMM's epilogue
-    } else if (ks > 1)
-      hipLaunchKernelGGL(reduce_rope_kernel, dim3(rows), dim3(256), 0, stream, g, ks, cs, sn, pos3, position, kc, vc,
-                         max_seq_len);
-    else
-      hipLaunchKernelGGL(rope_kv_kernel, dim3(rows), dim3(256), 0, stream, qkv, layer_weights, l, cs, sn, pos3, position,
-                         S, kc, vc, max_seq_len);
-    hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH), dim3(64 * AW), 0, stream, qkv, kc, vc, l, max_seq_len,
-                       position, S, att, scale, frag);
-    // O + residual, then the post-attention norm (fused with the split-K reduction)
-    g.A = att; g.lda = NQH * HDIM; g.N = kO.N; g.K = kO.K; g.out = h; g.ldo = HID; g.res = h; g.ldr = HID;
-    if ((ks = gemm<W_O, E_RESID>(g, stream, false)) == 0) return hipGetLastError();
-    if (ks > 1)
-      hipLaunchKernelGGL(reduce_resid_norm_kernel, dim3(rows), dim3(256), 0, stream, g, ks, l, 7, xn, frag);
-    else
-      hipLaunchKernelGGL(rmsnorm_kernel, dim3(norm_grid), dim3(256), 0, stream, h, HID, layer_weights, l, 7,
-                         (const bf16_t*)nullptr, xn, HID, (float*)nullptr, S, frag);
-    g.A = xn; g.lda = HID; g.N = kGU.N; g.K = kGU.K; g.out = act; g.ldo = INTER; g.res = nullptr;
-    if (gemm<W_GU, E_SWIGLU>(g, stream) == 0) return hipGetLastError();
-    // down + residual, then the next layer's input norm (fused with the split-K reduction)
-    const int nl = l + 1 < num_layers ? l + 1 : -1;
-    g.A = act; g.lda = INTER; g.N = kDown.N; g.K = kDown.K; g.out = h; g.ldo = HID; g.res = h; g.ldr = HID;
-    if ((ks = gemm<W_DOWN, E_RESID>(g, stream, false)) == 0) return hipGetLastError();
-    if (ks > 1)
-      hipLaunchKernelGGL(reduce_resid_norm_kernel, dim3(rows), dim3(256), 0, stream, g, ks, nl, 0, xn, frag);
-    else if (nl >= 0)
-      hipLaunchKernelGGL(rmsnorm_kernel, dim3(norm_grid), dim3(256), 0, stream, h, HID, layer_weights, nl, 0,
-                         (const bf16_t*)nullptr, xn, HID, (float*)nullptr, S, frag);
+    g.A = xg; g.out = q;
+    project_qkv(g, stream);
+    hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH), dim3(64 * AW), 0, stream, q, kc, vc, l, max_seq_len,
+                       position, S, att, scale);
+    g.A = att; g.nlayer = l; g.nfield = 7;
+    project_residual<P_O>(g, stream);
+    g.A = xg; g.out = act;
+    project_gate_up(g, stream);
+    g.A = act; g.nlayer = l + 1 < num_layers ? l + 1 : -1; g.nfield = 0;
+    project_residual<P_DOWN>(g, stream);
   }
-  // final norm of the last token -> hidden (bf16 values; f32 copy for the caller)
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(1), dim3(256), 0, stream, h + (size_t)(S - 1) * HID, HID,
-                     (const TTSLayerWeights*)nullptr, 0, 0, static_cast<const bf16_t*>(final_norm_weight), hb, HID,
-                     out_hidden, 1, 0);
+  // the last token's final norm -> hidden, and its logits
+  bf16_t* lg = reinterpret_cast<bf16_t*>(ws + L.logits);
+  const int head_grid = codec_head != nullptr ? (vocab + 4 * RPW - 1) / (4 * RPW) : 1;
+  hipLaunchKernelGGL(final_head_kernel, dim3(head_grid), dim3(256), 0, stream, h + (size_t)(S - 1) * HID,
+                     static_cast<const bf16_t*>(final_norm_weight), static_cast<const bf16_t*>(codec_head), vocab, out_hidden,
+                     lg);
   if (codec_head != nullptr) {
-    bf16_t* lg = reinterpret_cast<bf16_t*>(ws + L.logits);
-    GemmArgs g{};
-    g.A = hb; g.lda = HID; g.B = static_cast<const bf16_t*>(codec_head); g.M = 1; g.N = vocab; g.K = HID;
-    g.out = lg; g.ldo = vocab; g.part = part;
-    if (gemm<W_DIRECT, E_STORE>(g, stream) == 0) return hipGetLastError();
     SelParams sp{};
     sp.do_sample = sampling ? sampling->do_sample : 0;
     sp.temperature = sampling ? sampling->temperature : 1.0f;

@@ -25,24 +25,6 @@ __device__ __forceinline__ void best_merge(float& bv, int& bi, float ov, int oi)
   if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
 }
 
-// Greedy argmax over lg[0..n) (lowest index on ties; all -inf -> index 0), run by one wave.
-__device__ inline int wave_argmax(const float* lg, int n) {
-  const int lane = opaque((int)threadIdx.x & 63);
-  float best = -INFINITY;
-  int bi = 0x7fffffff;
-  for (int i = lane; i < n; i += 64) {
-    const float v = lg[i];
-    if (v > best || (v == best && i < bi)) { best = v; bi = i; }
-  }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
-  }
-  return bi == 0x7fffffff ? 0 : bi;
-}
-
 // LDS scratch of one selection: the short list (and a slot per lane for the writes that it does not
 // take); when more than SEL_CAP ids stay in the running, every logit and its probability (top-p).
 // Entries are words key << 16 | id.
@@ -308,20 +290,6 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
   return lo == 0x7fffffff ? 0 : lo;
 }
 
-// Selection over an LDS logit vector lg[0..n) (masked; bf16 values): greedy, or drawn.
-__device__ inline int wave_select(const float* lg, int n, const SelParams& sp, SelScratch* sc) {
-  if (!sp.do_sample) return wave_argmax(lg, n);
-  const int lane = opaque((int)threadIdx.x & 63);
-  uint32_t w[SEL_NJ];
-#pragma unroll
-  for (int j = 0; j < SEL_NJ; ++j) {
-    const int i = lane + 64 * j;
-    const uint32_t k = bfkey(lg[min(i, n - 1)]);
-    w[j] = i < n ? (k << 16) | (uint32_t)i : 0u;
-  }
-  return wave_sample(w, n, sp, sc);
-}
-
 // Selection from a head's logit slots, for the persistent decode kernels: n tagged slots at byte `off` of
 // the workspace polled straight into the key registers, masked, and drawn from (or the largest taken).
 // The kernels are instantiated apart for greedy and for sampled launches: with both selections in one
@@ -363,18 +331,24 @@ __device__ __forceinline__ void head_logits(const Poll& P, uint32_t off, int n, 
   part(std::integral_constant<int, 1>{});
   part(std::integral_constant<int, 2>{});
 }
-template <bool MASKED>
-__device__ __forceinline__ int head_argmax(const Poll& P, uint32_t off, int n, uint32_t tag, const HeadMask& hm,
-                                           const uint32_t* pen_bits) {
+// Greedy selection by words: larger value (-0 counts as +0, NaNs are passed over), then lower id.
+__device__ __forceinline__ uint32_t greedy_word(float x, int id) {
   static_assert(MAXV <= 4096, "12-bit ids");
-  uint32_t best = 0u;      // larger value, then lower id
-  head_logits<MASKED>(P, off, n, tag, hm, pen_bits, [&](int, int id, float x) QTTS_SEL_INLINE {
-    const uint32_t k = (bfkey(x != x ? -INFINITY : x + 0.0f) << 12) | (uint32_t)(4095 - id);
-    best = max(best, id < n ? k : 0u);
-  });
+  return (bfkey(x != x ? -INFINITY : x + 0.0f) << 12) | (uint32_t)(4095 - id);
+}
+__device__ __forceinline__ int greedy_id(uint32_t best, int n) {
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, o, 64));
   return min(4095 - (int)(best & 4095u), n - 1);
+}
+template <bool MASKED>
+__device__ __forceinline__ int head_argmax(const Poll& P, uint32_t off, int n, uint32_t tag, const HeadMask& hm,
+                                           const uint32_t* pen_bits) {
+  uint32_t best = 0u;
+  head_logits<MASKED>(P, off, n, tag, hm, pen_bits, [&](int, int id, float x) QTTS_SEL_INLINE {
+    best = max(best, id < n ? greedy_word(x, id) : 0u);
+  });
+  return greedy_id(best, n);
 }
 template <bool MASKED>
 __device__ __forceinline__ int head_sample(const Poll& P, uint32_t off, int n, uint32_t tag, const SelParams& sp,
