@@ -408,7 +408,7 @@ class MegakernelTTSDecoder {
   torch::Tensor k_cache_, v_cache_, hidden_buffer_, g_normalized_, logits_, token_, ws_;
   torch::Tensor ws_streams_;   // decode_steps_streams(): per-stream workspaces
   torch::Tensor ws_shared_;    // decode_steps_streams(shared=True): the weight-shared launches' workspace
-  torch::Tensor pf_ws_;        // prefill(): activations and split-K partials (grown on demand)
+  torch::Tensor pf_ws_;        // prefill(): activations (grown on demand)
 };
 
 // ---------------------------------------------------------------------------------------

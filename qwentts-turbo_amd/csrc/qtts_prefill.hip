@@ -26,11 +26,12 @@
 //   embed_kernel       the embeddings into the residual stream, layer 0's norm inputs
 //   tile_gemm_kernel   the four projections, K unsplit, with the norms, RoPE, K/V write, residual and SwiGLU
 //                      in their epilogues
-//   attn_kernel      causal GQA, 4 waves per (32-query block, query head) splitting the key
-//                    blocks: S^T = K Q^T on MFMA (each lane then holds one query's scores, so
-//                    the row max and sum stay in the lane and its partner half-wave), one pass
-//                    with a running max, O^T += V^T P^T on MFMA with V^T read from the row-major
-//                    V block through LDS transpose reads, partials merged in wave order
+//   attn_kernel        causal GQA, 4 waves per (32-query block, query head) splitting the key blocks: S^T = K
+//                      Q^T on MFMA (each lane then holds one query's scores, so the row max and sum stay in
+//                      the lane and its partner half-wave), one pass with a running max, O^T += V^T P^T on
+//                      MFMA with V^T read from the row-major V block through LDS transpose reads
+//   attn_pair_kernel   the same for long prompts: 8 waves per (32-query block, KV head), the two query heads
+//                      sharing each staged K and V block
 //   final_head_kernel  the last token's final norm and codec head
 //   select_kernel      suppress mask + EOS suppression + the decode kernels' selection
 #include <hip/hip_runtime.h>
@@ -156,7 +157,7 @@ constexpr int VROW = 160;     // LDS row of a staged V block (bf16): 320 B puts 
                               // transpose read touches 16 banks apart
 constexpr int WST = 32 * VROW;                      // a wave's staging region (K block, then V)
 constexpr int ATT_Q = 32 * QROW;                    // the query block
-constexpr int ATT_SMEM = std::max((ATT_Q + AW * WST) * 2, (AW - 1) * HDIM * 32 * 4 + AW * 2 * 32 * 4);
+constexpr int ATT_SMEM = std::max((ATT_Q + AW * WST) * 2, AW * HDIM * 32 * 4 + AW * 2 * 32 * 4);
 static_assert(32 * QROW <= WST, "a wave's LDS region holds its staged K block");
 
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -318,10 +319,11 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qrows, c
   }
   l += __shfl_xor(l, 32, 64);
 
-  // merge the waves: M = max m_w, L = sum l_w e^(m_w - M), O = sum O_w e^(m_w - M) (wave order)
+  // merge the waves: M = max m_w, L = sum l_w e^(m_w - M), O = sum O_w e^(m_w - M) (wave order), wave w
+  // finishing dims 32 w .. 32 w + 31 (one wave that merged and stored all of them took up to 1 us longer)
+  float* ob = reinterpret_cast<float*>(smem);   // [wave][dim block][register quad][lane][4]
+  float* sml = ob + AW * HDIM * 32;             // [AW][2][32]
   __syncthreads();   // every wave's staging region is dead
-  float* ob = reinterpret_cast<float*>(smem);
-  float* sml = ob + (AW - 1) * HDIM * 32;   // [AW][2][32]
   if (hf == 0) {
     sml[(w * 2) * 32 + c] = m;
     sml[(w * 2 + 1) * 32 + c] = l;
@@ -330,44 +332,38 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qrows, c
   float M = -INFINITY;
 #pragma unroll
   for (int v = 0; v < AW; ++v) M = fmaxf(M, sml[(v * 2) * 32 + c]);
-  const float sw = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * SL);
-  if (w > 0) {
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) ob[((w - 1) * 64 + mb * 16 + r) * 64 + lane] = o[mb][r] * sw;
-  }
-  __syncthreads();
-  if (w > 0 || !qok) return;
   float L = 0.0f;
 #pragma unroll
   for (int v = 0; v < AW; ++v) {
     const float mv = sml[(v * 2) * 32 + c];
     L += mv == -INFINITY ? 0.0f : sml[(v * 2 + 1) * 32 + c] * __builtin_amdgcn_exp2f((mv - M) * SL);
   }
+  const float sw = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * SL);
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[mb][r] *= sw;
-#pragma unroll 1
-  for (int v = 1; v < AW; ++v)
+    for (int r = 0; r < 4; ++r) {
+      f32x4 x;
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[mb][r] += ob[((v - 1) * 64 + mb * 16 + r) * 64 + lane];
+      for (int e = 0; e < 4; ++e) x[e] = o[mb][4 * r + e] * sw;
+      *reinterpret_cast<f32x4*>(ob + ((w * 4 + mb) * 4 + r) * 256 + lane * 4) = x;
+    }
+  __syncthreads();
+  if (!qok) return;
   const float rl = L > 0.0f ? 1.0f / L : 0.0f;
   // O^T layout: column = query c, register r of block mb = dim 32 mb + 8 (r >> 2) + 4 hf + (r & 3)
-  const size_t orow = (size_t)i * (NQH * HDIM) + hq * HDIM;
+  static_assert(AW == 4, "a dim block per wave");
+  bf16_t* orow = att + (size_t)i * (NQH * HDIM) + hq * HDIM + 32 * w + 4 * hf;
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int r = 0; r < 4; ++r) {
+    f32x4 x = *reinterpret_cast<const f32x4*>(ob + (w * 4 + r) * 256 + lane * 4);
 #pragma unroll
-    for (int rq = 0; rq < 4; ++rq) {
-      const int d0 = 32 * mb + 8 * rq + 4 * hf;
-      u32x2 pk;
-      pk[0] = pack_bh(o[mb][4 * rq] * rl, o[mb][4 * rq + 1] * rl);
-      pk[1] = pack_bh(o[mb][4 * rq + 2] * rl, o[mb][4 * rq + 3] * rl);
-      *reinterpret_cast<u32x2*>(att + orow + d0) = pk;
-    }
+    for (int v = 1; v < AW; ++v) x += *reinterpret_cast<const f32x4*>(ob + ((v * 4 + w) * 4 + r) * 256 + lane * 4);
+    u32x2 pk;
+    pk[0] = pack_bh(x[0] * rl, x[1] * rl);
+    pk[1] = pack_bh(x[2] * rl, x[3] * rl);
+    *reinterpret_cast<u32x2*>(orow + 8 * r) = pk;
+  }
 }
 
 // Wait until at most N of this wave's vector-memory instructions are in flight (the compiler does not
@@ -383,6 +379,243 @@ template <int N>
 __device__ __forceinline__ void wait_vm_lds() {
   static_assert(N >= 0 && N <= 63, "vmcnt field");
   __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+}
+
+// The same attention for long prompts, one workgroup of 8 waves per (32-query block, KV head): wave (hd, ks) takes query head 2 kvh + hd and the 32-key
+// blocks kb = ks, ks + 4, ... in one pass with a running (online) softmax. The two heads of a KV head share
+// each staged K and V block, and the queries stay in registers, so that a wave's 32 x 32 block costs 24 KB of
+// LDS traffic (40 KB in attn_kernel). 47 -> 38 us at 2048 tokens, 18.7 -> 16.8 at 1000.
+// What bounds it now is the chain of a step (1.6 us: wait and barrier 0.4, copies issued 0.3, scores, softmax and
+// P V 0.3 each) at two waves a SIMD: taking the next block's scores under this one's softmax, or staging through
+// registers two steps ahead, changed nothing.
+//   * K and V blocks (32 keys x 128 dims) come by DMA into the pair's two buffers, one step ahead; chunk c
+//     (16 bytes) of row r sits at position c ^ (r & 7).
+//   * The layouts of S^T, P and O^T are attn_kernel's; O^T and l are rescaled only when some query's block
+//     max passes the running one by more than 2^8.
+// The key splits of a
+// head merge through LDS in split order, wave ks finishing dims 32 ks .. 32 ks + 31. Workgroups: KV head =
+// linear id mod 8 (one head per XCD's L2), the longest query blocks first.
+constexpr int AKS = 4;                              // key splits
+constexpr int ABLK = 32 * HDIM * 2;                 // bytes of a K or V block
+constexpr int ATTP_SMEM = AKS * 2 * 2 * ABLK + 2 * AKS * 2 * 32 * 4;   // (K, V) x 2 buffers per split; (m, l) of the merge
+
+// The 8 transpose reads of a 16-key step: the low and high 4 keys of 4 dim blocks at LDS addresses a[0..3],
+// OFF bytes further. In assembly, with their wait: before the builtin the compiler waits for every DMA in
+// flight, the next block's among them (it takes any of them for the read's source).
+template <int OFF>
+__device__ __forceinline__ void lds_tr16x8(const uint32_t (&a)[4], u32x2 (&lo)[4], u32x2 (&hi)[4]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8 offset:%c12\n\tds_read_b64_tr_b16 %4, %8 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %1, %9 offset:%c12\n\tds_read_b64_tr_b16 %5, %9 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %2, %10 offset:%c12\n\tds_read_b64_tr_b16 %6, %10 offset:%c13\n\t"
+      "ds_read_b64_tr_b16 %3, %11 offset:%c12\n\tds_read_b64_tr_b16 %7, %11 offset:%c13\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(hi[0]), "=&v"(hi[1]), "=&v"(hi[2]), "=&v"(hi[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "i"(OFF), "i"(OFF + 8 * HDIM * 2)
+      : "memory");
+}
+
+__global__ void __launch_bounds__(128 * AKS, 2) attn_pair_kernel(const bf16_t* qrows, const bf16_t* kc, const bf16_t* vc,
+                                                            int layer, int max_seq, int p0, int S, bf16_t* att, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[ATTP_SMEM];   // (one LDS object, as in tile_gemm_kernel)
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int hd = w & 1, ks = w >> 1, hf = lane >> 5, c = lane & 31;
+  const int nqb = (S + 31) / 32, id = blockIdx.x;
+  const int kvh = id & 7, qb = nqb - 1 - (id >> 3);
+  const int hq = 2 * kvh + hd;
+  const int i = 32 * qb + c;
+  const bool qok = i < S;
+  const int last = p0 + min(S, 32 * qb + 32) - 1;   // last key any query of the block sees
+  const int nkb = last / 32 + 1, nst = (nkb + AKS - 1) / AKS;
+  const size_t hbase = ((size_t)layer * NKVH + kvh) * max_seq * HDIM;
+
+  // wave (hd, ks) copies rows 16 hd .. 16 hd + 15 of the split's K block and of its V block, 4 rows an
+  // instruction, through buffer descriptors that end after row `last`: rows past it come as zeros (their
+  // scores are masked), and a step moves one scalar offset, no vector address
+  char* const buf = smem + ks * 4 * ABLK;
+  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(kc + hbase), (short)0,
+                                                                       (last + 1) * HDIM * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vc + hbase), (short)0,
+                                                                       (last + 1) * HDIM * 2, 0x00020000);
+  const int drow = 16 * hd + (lane >> 4);
+  int doff[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) doff[r] = (drow + 4 * r) * HDIM * 2 + ((lane & 15) ^ ((drow + 4 * r) & 7)) * 16;
+  auto issue = [&](int b, int kb) QTTS_PF_INLINE {
+    const int so = min(kb, nkb - 1) * ABLK;   // inside the descriptor: only the rows of a block can pass its end
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      char* dst = buf + b * 2 * ABLK + (16 * hd + 4 * r) * HDIM * 2;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lvoid_t*)dst, 16, doff[r], so, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lvoid_t*)(dst + ABLK), 16, doff[r], so, 0, 0);
+    }
+  };
+  // e^(scale (s - m)) as 2^(s scale log2 e - m scale log2 e): one fma into the hardware exp2
+  const float SL = scale * 1.4426950408889634f;
+  auto ex = [SL](float s, float nm) QTTS_PF_INLINE { return __builtin_amdgcn_exp2f(fmaf(s, SL, nm)); };
+
+  float m = -INFINITY, l = 0.0f;
+  f32x16 o[4];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[mb][r] = 0.0f;
+  // LDS offsets of this lane: K row c (chunk 2 kk + hf), and the transpose reads of V (row vr, chunk
+  // 4 mb + vch, 8 bytes at vin; rows 8 and 16 further have the same swizzle)
+  const int gi = lane & 15, gg = lane >> 4;
+  const int vrow = 4 * (gg >> 1) + (gi >> 2), vch = 2 * (gg & 1) + ((gi & 3) >> 1), vin = 8 * (gi & 1);
+  uint32_t vaddr[4];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+    vaddr[mb] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)buf + ABLK + vrow * HDIM * 2 +
+                ((4 * mb + vch) ^ (vrow & 7)) * 16 + vin;
+
+  // the two heads' 32 query rows come by DMA too, into the split-0 buffer that the second step fills (read
+  // in operand order from memory, 16 rows an instruction, they kept the address unit busy for 1.9 us), head
+  // h's into block h; then every wave takes its own, the B operand: query c, dims 16 kk + 8 hf ..
+  char* const qbuf = smem + 2 * ABLK;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int row = 8 * ks + 4 * r + (lane >> 4);
+    const bf16_t* src = qrows + (size_t)min(32 * qb + row, S - 1) * (NQH * HDIM) + hq * HDIM + ((lane & 15) ^ (row & 7)) * 8;
+    __builtin_amdgcn_global_load_lds((gvoid_t*)src, (lvoid_t*)(qbuf + hd * ABLK + (8 * ks + 4 * r) * HDIM * 2), 16, 0, 0);
+  }
+  issue(0, ks);
+  wait_vm_lds<0>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  u32x4 q[8];
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk)
+    q[kk] = *reinterpret_cast<const u32x4*>(qbuf + hd * ABLK + c * HDIM * 2 + ((2 * kk + hf) ^ (c & 7)) * 16);
+#pragma unroll 1
+  for (int t = 0; t < nst; ++t) {
+    const int kb = ks + AKS * t, b = t & 1;
+    wait_vm_lds<0>();                 // this wave's copies have landed, its reads of the other buffer are done
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");    // no LDS access moves across
+    issue(b ^ 1, kb + AKS);           // (past the end: the last block again, which nothing reads)
+    if (kb >= nkb) continue;
+    const char* K = buf + b * 2 * ABLK;
+    u32x4 kf[8];
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      kf[kk] = *reinterpret_cast<const u32x4*>(K + c * HDIM * 2 + ((2 * kk + hf) ^ (c & 7)) * 16);
+    f32x16 acc, acc2;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = acc2[r] = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < 8; kk += 2) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(kf[kk]), as_bf8(q[kk]), acc, 0, 0, 0);
+      acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(kf[kk + 1]), as_bf8(q[kk + 1]), acc2, 0, 0, 0);
+    }
+    float sc[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sc[r] = acc[r] + acc2[r];
+    // blocks that every query of the block sees whole (the wave-uniform common case) skip the mask
+    if (!(32 * kb + 31 <= p0 + 32 * qb && 32 * qb + 31 < S)) {
+      const int lim = qok ? p0 + i : -1;   // last key this lane's query sees (none past the prompt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * kb + 8 * (r >> 2) + 4 * hf + (r & 3) > lim) sc[r] = -INFINITY;
+    }
+    // running max; a fully masked row so far keeps m = -inf and adds nothing. It moves only when some
+    // query's block max passes it by more than a factor 2^8 of the weights (p <= 256 keeps its relative
+    // rounding, and the sums are f32), so that most steps do not rescale O^T
+    // (v_max3 by name: fmaxf first quiets each operand)
+    float bm = sc[0];
+    auto max3 = [](float x, float y, float z) QTTS_PF_INLINE {
+      float r;
+      asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
+      return r;
+    };
+    {
+      const float x0 = max3(sc[0], sc[1], sc[2]), x1 = max3(sc[3], sc[4], sc[5]), x2 = max3(sc[6], sc[7], sc[8]);
+      const float x3 = max3(sc[9], sc[10], sc[11]), x4 = max3(sc[12], sc[13], sc[14]);
+      bm = max3(max3(x0, x1, sc[15]), x2, max3(x3, x4, x4));
+    }
+    bm = fmaxf(bm, __uint_as_float(xlane<5>(__float_as_uint(bm))));
+    if (__builtin_amdgcn_ballot_w64(bm > m + 8.0f / SL) != 0ull) {
+      const float mn = fmaxf(m, bm);
+      const float al = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * SL);
+      l *= al;
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[mb][r] *= al;
+      m = mn;
+    }
+    const float nm = m == -INFINITY ? 0.0f : -m * SL;
+    float e[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) e[r] = ex(sc[r], nm);
+    l += (((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]))) +
+         (((e[8] + e[9]) + (e[10] + e[11])) + ((e[12] + e[13]) + (e[14] + e[15])));
+    uint32_t va[4];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) va[mb] = vaddr[mb] + b * 2 * ABLK;
+    auto pv = [&](auto kk_) QTTS_PF_INLINE {
+      constexpr int kk2 = decltype(kk_)::value;
+      u32x4 pb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pb[j] = pack_bh(e[8 * kk2 + 2 * j], e[8 * kk2 + 2 * j + 1]);
+      u32x2 lo[4], hi[4];
+      lds_tr16x8<16 * kk2 * HDIM * 2>(va, lo, hi);
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        const u32x4 av = {lo[mb][0], lo[mb][1], hi[mb][0], hi[mb][1]};
+        o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(av), as_bf8(pb), o[mb], 0, 0, 0);
+      }
+    };
+    pv(std::integral_constant<int, 0>{});
+    pv(std::integral_constant<int, 1>{});
+  }
+  l += __uint_as_float(xlane<5>(__float_as_uint(l)));
+
+  // merge the splits: M = max m_s, L = sum l_s e^(m_s - M), O = sum O_s e^(m_s - M) (split order)
+  float* sml = reinterpret_cast<float*>(smem + AKS * 4 * ABLK) + hd * AKS * 2 * 32;   // [split][2][32]
+  if (hf == 0) {
+    sml[(ks * 2) * 32 + c] = m;
+    sml[(ks * 2 + 1) * 32 + c] = l;
+  }
+  wait_vm_lds<0>();
+  __syncthreads();   // every buffer is dead
+  float M = -INFINITY;
+#pragma unroll
+  for (int v = 0; v < AKS; ++v) M = fmaxf(M, sml[(v * 2) * 32 + c]);
+  float L = 0.0f;
+#pragma unroll
+  for (int v = 0; v < AKS; ++v) {
+    const float mv = sml[(v * 2) * 32 + c];
+    L += mv == -INFINITY ? 0.0f : sml[(v * 2 + 1) * 32 + c] * __builtin_amdgcn_exp2f((mv - M) * SL);
+  }
+  const float sw = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * SL);
+  // part [head][split][32 dims][64 lanes]: wave ks leaves its sums of the dims that another wave finishes
+  float* ob = reinterpret_cast<float*>(smem) + hd * AKS * 64 * 64;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      f32x4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = o[mb][4 * r + e] * sw;
+      *reinterpret_cast<f32x4*>(ob + ((ks * 4 + mb) * 4 + r) * 256 + lane * 4) = x;
+    }
+  __syncthreads();
+  if (!qok) return;
+  const float rl = L > 0.0f ? 1.0f / L : 0.0f;
+  // O^T layout: column = query c, register r of block mb = dim 32 mb + 8 (r >> 2) + 4 hf + (r & 3)
+  bf16_t* orow = att + (size_t)i * (NQH * HDIM) + hq * HDIM + 32 * ks + 4 * hf;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    f32x4 x = *reinterpret_cast<const f32x4*>(ob + (ks * 4 + r) * 256 + lane * 4);
+#pragma unroll
+    for (int v = 1; v < AKS; ++v) x += *reinterpret_cast<const f32x4*>(ob + ((v * 4 + ks) * 4 + r) * 256 + lane * 4);
+    u32x2 pk;
+    pk[0] = pack_bh(x[0] * rl, x[1] * rl);
+    pk[1] = pack_bh(x[2] * rl, x[3] * rl);
+    *reinterpret_cast<u32x2*>(orow + 8 * r) = pk;
+  }
 }
 
 // Layer projection C = A W^T of a TM x TN tile (tokens x weight rows), the whole K range in one
@@ -998,8 +1231,16 @@ hipError_t qtts_backbone_prefill(void* workspace, size_t workspace_bytes, const 
     g.layer = l;
     g.A = xg; g.out = q;
     project_qkv(g, stream);
-    hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH), dim3(64 * AW), 0, stream, q, kc, vc, l, max_seq_len,
-                       position, S, att, scale);
+    // the two-head kernel from where its workgroups, half as many, come near one a CU (us a layer, per head
+    // against two heads: 512 tokens 61.2 : 61.5, 640 75.4 : 75.2, 768 77.1 : 76.8, 1000 82.9 : 81.9, 2048
+    // 147 : 138, 3000 259 : 247; with a prefix before the prompt 333 after 1500 71.7 : 75.9, 768 after 1500
+    // 96.2 : 95.4, 2048 after 1500 190 : 172)
+    if ((S + 31) / 32 * NKVH >= 192)
+      hipLaunchKernelGGL(attn_pair_kernel, dim3((S + 31) / 32 * NKVH), dim3(128 * AKS), 0, stream, q, kc, vc, l, max_seq_len,
+                         position, S, att, scale);
+    else
+      hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH), dim3(64 * AW), 0, stream, q, kc, vc, l, max_seq_len,
+                         position, S, att, scale);
     g.A = att; g.nlayer = l; g.nfield = 7;
     project_residual<P_O>(g, stream);
     g.A = xg; g.out = act;
