@@ -400,9 +400,9 @@ def main():
     t_bb = sum(e[1].elapsed_time(e[2]) for e in ev) / n_ev * 1e-3
     cp_gbs = cp_frame_bytes() / t_cp / 1e9
     bb_gbs = backbone_bytes(512) / t_bb / 1e9
-    dominant = ("qtts_decode_kernel<false, false> (code-predictor frame)", cp_gbs, cp_frame_bytes(), PMC_TRAFFIC["cp_frame"]) \
+    dominant = ("qtts_decode_kernel<false, false, false> (code-predictor frame)", cp_gbs, cp_frame_bytes(), PMC_TRAFFIC["cp_frame"]) \
         if t_cp >= t_bb else \
-        ("qtts_decode_kernel<true, false> (backbone step, L=512)", bb_gbs, backbone_bytes(512), PMC_TRAFFIC["backbone_step"])
+        ("qtts_decode_kernel<true, false, false> (backbone step, L=512)", bb_gbs, backbone_bytes(512), PMC_TRAFFIC["backbone_step"])
 
     fps = args.steps / el
     out = {

@@ -274,7 +274,7 @@ hipError_t qtts_backbone_step_streams(
  * [num_layers, 8, max_seq_len, 128], the decode layout); attention covers cache positions
  * 0 .. position + n_tokens - 1 (causal), so a prefix already in the cache is attended.
  * Arithmetic follows the transformers bf16 forward (bf16 storage after every op, f32 sums on
- * bf16 MFMA). pos3: NULL (t = h = w = position of the token) or device int32 [3][n_tokens]
+ * bf16 MFMA; the layer norms' rstd scales the f32 sums of the projection after them). pos3: NULL (t = h = w = position of the token) or device int32 [3][n_tokens]
  * rotary (t, h, w) rows of the bf16 tables (clamped to [0, max_seq_len)). out_hidden: f32 [1024],
  * the final-norm hidden of the last token (bf16 values). When codec_head is not NULL the first
  * group-0 token is selected from bf16(codec_head . hidden) as in generator.py:113-119 (suppress
