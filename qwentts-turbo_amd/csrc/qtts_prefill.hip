@@ -29,7 +29,8 @@
 //   attn_kernel        causal GQA, 4 waves per (32-query block, query head) splitting the key blocks: S^T = K
 //                      Q^T on MFMA (each lane then holds one query's scores, so the row max and sum stay in
 //                      the lane and its partner half-wave), one pass with a running max, O^T += V^T P^T on
-//                      MFMA with V^T read from the row-major V block through LDS transpose reads
+//                      MFMA with V^T read from the row-major V block through LDS transpose reads; further
+//                      workgroups read the weights of the launches that follow
 //   attn_pair_kernel   the same for long prompts: 8 waves per (32-query block, KV head), the two query heads
 //                      sharing each staged K and V block
 //   final_head_kernel  the last token's final norm and codec head
@@ -167,9 +168,44 @@ __device__ __forceinline__ u32x2 lds_tr16(const bf16_t* p) {
   return __builtin_bit_cast(u32x2, r);
 }
 
+// The weights that follow the attention are read while it runs: attn_kernel leaves most of the memory system
+// idle, and the projections after it would wait for each line to come from HBM. A workgroup reads one 16 KB
+// piece (64 bytes a thread) of the layer's O, gate, up and down weights and of the next layer's q, k and v,
+// into the memory-side cache. Us a layer over 28 layers without and with: 13 tokens 37.9 : 34.3, 64 40.1 : 35.9,
+// 128 40.0 : 36.8, 200 42.9 : 41.4, 333 56.3 : 53.7, 512 60.1 : 55.8, 700 76.0 : 70.9 (without the next layer's
+// 0.4 to 0.9 more; 192 workgroups that share the pieces 1 to 3 more). Done by the projections themselves for
+// their own operands it was slower.
+constexpr int PIECE = 16384;
+constexpr int kPiecesSq = HID * NQH * HDIM * 2 / PIECE, kPiecesKv = kPiecesSq / 2, kPiecesMlp = INTER * HID * 2 / PIECE;
+constexpr int kPiecesLayer = kPiecesSq + 3 * kPiecesMlp, kPiecesNext = kPiecesSq + 2 * kPiecesKv;
+static_assert(64 * AW * 64 == PIECE, "64 bytes a thread");
+__device__ __forceinline__ void weight_piece_ahead(const TTSLayerWeights* lw, int u) {
+  int field = 6;                                        // O
+  if (u >= kPiecesLayer) {
+    u -= kPiecesLayer;
+    ++lw;
+    field = u < kPiecesSq ? 1 : (u < kPiecesSq + kPiecesKv ? 2 : 3);
+    u -= field == 1 ? 0 : (field == 2 ? kPiecesSq : kPiecesSq + kPiecesKv);
+  } else if (u >= kPiecesSq) {
+    u -= kPiecesSq;
+    field = 8 + u / kPiecesMlp;
+    u %= kPiecesMlp;
+  }
+  const bf16_t* p = tbl(lw, field) + (size_t)u * (PIECE / 2);
+  u32x4 v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = ldw(p + (threadIdx.x + 64 * AW * r) * 8);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) asm volatile("" ::"v"(v[r]));   // (keeps the loads)
+}
+
 __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qrows, const bf16_t* kc, const bf16_t* vc,
                                                        int layer, int max_seq, int p0, int S, bf16_t* att,
-                                                       float scale) {
+                                                       float scale, const TTSLayerWeights* layers) {
+  if ((int)blockIdx.x >= (S + 31) / 32 * NQH) {   // workgroups past the queries'
+    weight_piece_ahead(layers + layer, (int)blockIdx.x - (S + 31) / 32 * NQH);
+    return;
+  }
   __shared__ __attribute__((aligned(16))) char smem[ATT_SMEM];
   bf16_t* sq = reinterpret_cast<bf16_t*>(smem);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, hf = lane >> 5, c = lane & 31;
@@ -1232,16 +1268,17 @@ hipError_t qtts_backbone_prefill(void* workspace, size_t workspace_bytes, const 
     g.layer = l;
     g.A = xg; g.out = q;
     project_qkv(g, stream);
-    // the two-head kernel from where its workgroups, half as many, come near one a CU (us a layer, per head
-    // against two heads: 512 tokens 61.2 : 61.5, 640 75.4 : 75.2, 768 77.1 : 76.8, 1000 82.9 : 81.9, 2048
-    // 147 : 138, 3000 259 : 247; with a prefix before the prompt 333 after 1500 71.7 : 75.9, 768 after 1500
-    // 96.2 : 95.4, 2048 after 1500 190 : 172)
-    if ((S + 31) / 32 * NKVH >= 192)
+    // the two-head kernel for prompts that fill the chip with half the workgroups; below, the per-head kernel
+    // and its reads ahead (us a layer, per head against two heads: 640 tokens 69.2 : 75.2, 768 72.0 : 76.9,
+    // 1000 79.4 : 81.6, 1280 111.1 : 116.2, 1500 117.0 : 118.4, 2048 141.5 : 137.4, 3000 248.2 : 246.4; with a
+    // prefix before the prompt 768 after 1500 90.3 : 95.3, 1000 after 2000 106.8 : 106.4, 1500 after 1500
+    // 151.2 : 150.4, 2048 after 1500 181.3 : 170.1)
+    if ((S + 31) / 32 * NKVH >= 448)
       hipLaunchKernelGGL(attn_pair_kernel, dim3((S + 31) / 32 * NKVH), dim3(128 * AKS), 0, stream, q, kc, vc, l, max_seq_len,
                          position, S, att, scale);
     else
-      hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH), dim3(64 * AW), 0, stream, q, kc, vc, l, max_seq_len,
-                         position, S, att, scale);
+      hipLaunchKernelGGL(attn_kernel, dim3((S + 31) / 32 * NQH + kPiecesLayer + (l + 1 < num_layers ? kPiecesNext : 0)),
+                         dim3(64 * AW), 0, stream, q, kc, vc, l, max_seq_len, position, S, att, scale, layer_weights);
     g.A = att; g.nlayer = l; g.nfield = 7;
     project_residual<P_O>(g, stream);
     g.A = xg; g.out = act;

@@ -52,7 +52,7 @@ def model(pkg):
 @pytest.mark.parametrize("tokens,prefix,distinct", [
     (1, 0, False), (15, 0, False), (16, 3, True), (17, 0, False), (32, 0, False), (33, 31, True), (128, 0, False), (129, 0, True),
     (256, 32, False), (257, 0, False), (512, 0, False), (513, 700, True), (736, 0, False), (737, 0, False), (737, 1000, True),
-    (1024, 0, False), (1025, 0, False), (2049, 0, False)])
+    (1024, 0, False), (1025, 0, False), (1760, 0, False), (1761, 300, True), (2049, 0, False)])
 def test_prefill_at_tile_edges(model, tokens, prefix, distinct):
     sd, bb = model
     g = torch.Generator(device="cuda").manual_seed(tokens + prefix)
