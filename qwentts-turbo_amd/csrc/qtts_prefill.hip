@@ -1144,7 +1144,7 @@ void launch_tile(TileArgs& g, hipStream_t st) {
 
 // Tiles by prompt length M. A projection's time is its workgroups' K loop (operand bytes per CU through
 // LDS) plus about 4 us of launch, first loads and epilogue, so the tile grows with M as slowly as 256
-// workgroups, one a CU, allow. Measured over prompts of 13 to 2048 tokens (us a layer, against the best
+// workgroups, one a CU, allow. Measured over prompts of 13 to 2048 tokens, without reads ahead (us a layer, against the best
 // alternative):
 //   QKV (a head's 128 columns)  32 tokens up to 256, 64 to 512, 128 to 1024, then 256; a step too small
 //                               or too large costs 2 to 10 us
