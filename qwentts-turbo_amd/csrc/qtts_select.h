@@ -35,8 +35,8 @@ struct SelScratch {
   double p[MAXV];
 };
 
-// Order-preserving 16-bit key of a bf16 value and back (-inf is SEL_NINF; NaNs lie outside).
-constexpr uint32_t SEL_NINF = 0x007fu;
+// Order-preserving 16-bit key of a bf16 value and back (-inf is SEL_NINF, +inf SEL_PINF; NaNs lie outside, by their sign).
+constexpr uint32_t SEL_NINF = 0x007fu, SEL_PINF = 0xff80u;
 __device__ __forceinline__ uint32_t bfkey(float f) { return fkey(f) >> 16; }
 __device__ __forceinline__ float bfkey_value(uint32_t k) {
   return __uint_as_float(((k & 0x8000u) ? (k ^ 0x8000u) : (k ^ 0xffffu)) << 16);
@@ -77,6 +77,17 @@ __device__ __forceinline__ uint32_t sel_kth(const uint32_t (&w)[N], int k) {
     if (c >= k) t = cand;
   }
   return t >> 16;
+}
+
+// Greedy selection by words: larger value (-0 counts as +0, a NaN is below -inf), then lower id.
+__device__ __forceinline__ uint32_t greedy_word(float x, int id) {
+  static_assert(MAXV <= 4096, "12-bit ids");
+  return (x != x ? 0u : bfkey(x + 0.0f) << 12) | (uint32_t)(4095 - id);
+}
+__device__ __forceinline__ int greedy_id(uint32_t best, int n) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, o, 64));
+  return min(4095 - (int)(best & 4095u), n - 1);
 }
 
 // Temperature / top-k / top-p / Gumbel-max over n <= MAXV masked logits (bf16 values; suppressed ids
@@ -276,15 +287,18 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
   merge(xlane_d<5>(best), (int)xlane<5>((uint32_t)bi));
   bi = __builtin_amdgcn_readfirstlane(bi);
   if (bi != 0x7fffffff) return bi;
-  // nothing to draw from (every id suppressed): the largest logit, the lowest id on ties
+  // nothing to draw from (every id suppressed, or a probability mass that is no number): the largest logit, the
+  // lowest id on ties (-0 counts as +0). Keys above +inf's are NaNs'.
+  const int nans = count(SEL_PINF + 1u);
   uint32_t bk = 0u;
 #pragma unroll 1
   for (int b = 15; b >= 0; --b)
-    if (count(bk | (1u << b)) >= 1) bk |= 1u << b;
+    if (count(bk | (1u << b)) > nans) bk |= 1u << b;
+  const uint32_t tie = bk == 0x8000u ? 0x7fffu : bk;
   int lo = 0x7fffffff;
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
-    if (w[j] >> 16 == bk && bk != 0u) lo = min(lo, (int)(w[j] & 0xffffu));
+    if ((w[j] >> 16) - tie <= bk - tie && bk >= SEL_NINF) lo = min(lo, (int)(w[j] & 0xffffu));
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) lo = min(lo, __shfl_xor(lo, o, 64));
   return lo == 0x7fffffff ? 0 : lo;
@@ -330,16 +344,6 @@ __device__ __forceinline__ void head_logits(const Poll& P, uint32_t off, int n, 
   part(std::integral_constant<int, 0>{});
   part(std::integral_constant<int, 1>{});
   part(std::integral_constant<int, 2>{});
-}
-// Greedy selection by words: larger value (-0 counts as +0, NaNs are passed over), then lower id.
-__device__ __forceinline__ uint32_t greedy_word(float x, int id) {
-  static_assert(MAXV <= 4096, "12-bit ids");
-  return (bfkey(x != x ? -INFINITY : x + 0.0f) << 12) | (uint32_t)(4095 - id);
-}
-__device__ __forceinline__ int greedy_id(uint32_t best, int n) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, o, 64));
-  return min(4095 - (int)(best & 4095u), n - 1);
 }
 template <bool MASKED>
 __device__ __forceinline__ int head_argmax(const Poll& P, uint32_t off, int n, uint32_t tag, const HeadMask& hm,
