@@ -227,8 +227,10 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
         if (count(thr | (1u << b)) >= sp.top_k) thr |= 1u << b;
       thr = sel_lowest_tie(thr, T);
     }
+    // a NaN that is kept makes the mass under top-p no number, also one with its sign bit set (below -inf)
+    const bool no_mass = sp.top_p < 1.0f && thr < SEL_NINF && (thr == 0u ? n : count(thr)) > count(SEL_NINF);
     thr = max(thr, SEL_NINF + 1u);         // suppressed ids are never drawn
-    const int c = collect(thr);
+    const int c = no_mass ? 0 : collect(thr);
     if (c <= SEL_CAP) {
       n_in = finish_list(c, 0);
     } else {

@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 
 EOS, VOCAB, CP_VOCAB, GROUPS, STEP, SEED = 2150, 3072, 2048, 15, 6, 4242
 INF = float("inf")
-DESIGNS = ("plain", "nan", "nan_none", "inf", "few", "none", "ties", "wide")
+DESIGNS = ("plain", "nan", "nan_neg", "nan_none", "inf", "few", "none", "ties", "wide")
 
 
 def _logits(design, n, seed):
@@ -29,9 +29,9 @@ def _logits(design, n, seed):
     if design == "nan_none":                    # NaN or -inf
         w = torch.full((n,), -3e38).to(torch.bfloat16)
         w.view(torch.int16)[[0, 7]] = 0x7FC0
-    elif design == "nan":
+    elif design in ("nan", "nan_neg"):
         at, w = torch.randperm(n, generator=g)[:3], w.to(torch.bfloat16)
-        w.view(torch.int16)[at] = 0x7FC0
+        w.view(torch.int16)[at] = 0x7FC0 if design == "nan" else -0x40
     elif design == "inf":                       # 32 w overflows
         w[torch.randperm(2000, generator=g)[:5]] = torch.tensor([3e38, 3e38, -3e38, -3e38, 3e38])
     elif design == "few":
@@ -216,8 +216,8 @@ def test_every_entry_point(models, design, temperature, top_k, top_p):
     _both(models, design, temperature, top_k, top_p)
 
 
-@pytest.mark.parametrize("temperature,top_k,top_p", [s for s in SETTINGS if s != (0.9, 0, 0.5)])
-@pytest.mark.parametrize("design", ["nan", "nan_none"])
+@pytest.mark.parametrize("temperature,top_k,top_p", SETTINGS)
+@pytest.mark.parametrize("design", ["nan", "nan_neg", "nan_none"])
 def test_nan_logits_are_passed_over(models, design, temperature, top_k, top_p):
     """A NaN never wins, and where it leaves nothing to draw from (top_k = 1, or top-p over a mass that is no
     number) the largest of the other logits is taken."""
