@@ -201,8 +201,9 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
   };
 
   const bool limited = sp.top_k > 0 && sp.top_k < n;
+  const bool reversed = __builtin_signbit(T);   // the scaled values fall as the keys rise: everything on scaled words
   int n_in = -1;                           // words to draw from, in the list or (more than SEL_CAP) in `all`
-  if (limited && sp.top_k <= 64) {
+  if (limited && sp.top_k <= 64 && !reversed) {
     uint32_t lmax[1] = {0u};
 #pragma unroll
     for (int j = 0; j < NJ; ++j) lmax[0] = max(lmax[0], w[j]);
@@ -221,16 +222,16 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
   }
   if (n_in < 0) {
     uint32_t thr = 0u;                     // the lowest logit key that top-k keeps
-    if (limited) {
+    if (limited && !reversed) {
 #pragma unroll 1
       for (int b = 15; b >= 0; --b)
         if (count(thr | (1u << b)) >= sp.top_k) thr |= 1u << b;
       thr = sel_lowest_tie(thr, T);
     }
     // a NaN that is kept makes the mass under top-p no number, also one with its sign bit set (below -inf)
-    const bool no_mass = sp.top_p < 1.0f && thr < SEL_NINF && (thr == 0u ? n : count(thr)) > count(SEL_NINF);
-    thr = max(thr, SEL_NINF + 1u);         // suppressed ids are never drawn
-    const int c = no_mass ? 0 : collect(thr);
+    const bool no_mass = !reversed && sp.top_p < 1.0f && thr < SEL_NINF && (thr == 0u ? n : count(thr)) > count(SEL_NINF);
+    thr = max(thr, reversed ? 0u : SEL_NINF + 1u);   // suppressed ids are never drawn
+    const int c = reversed ? SEL_CAP + 1 : (no_mass ? 0 : collect(thr));
     if (c <= SEL_CAP) {
       n_in = finish_list(c, 0);
     } else {
@@ -241,7 +242,21 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
       for (int i = lane; i < MAXV; i += 64) {
         const uint32_t e = sc->all[i];
         const float v = sel_scaled(e >> 16, T);
-        sc->all[i] = e >= (thr << 16) && v != -INFINITY ? (bfkey(v) << 16) | (e & 0xffffu) : 0u;
+        sc->all[i] = e != 0u && e >= (thr << 16) && v != -INFINITY ? (bfkey(v) << 16) | (e & 0xffffu) : 0u;
+      }
+      if (reversed && limited) {
+        uint32_t k = 0u;
+#pragma unroll 1
+        for (int b = 15; b >= 0; --b) {
+          const uint32_t cand = k | (1u << b);
+          int kept = 0;
+#pragma unroll 1
+          for (int i = lane; i < MAXV; i += 64) kept += __popcll(__ballot(sc->all[i] >= (cand << 16)));
+          if (kept >= sp.top_k) k = cand;
+        }
+#pragma unroll 1
+        for (int i = lane; i < MAXV; i += 64)
+          if (sc->all[i] < (k << 16)) sc->all[i] = 0u;
       }
       n_in = MAXV;
       if (sp.top_p < 1.0f) {

@@ -14,7 +14,7 @@ import struct
 import pytest
 import torch
 
-from oracle.qtts_oracle import DecoderOracle, TalkerWeights, rel_l2, rope_tables
+from oracle.qtts_oracle import DecoderOracle, TalkerWeights, rel_l2, rope_tables, sample_token
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
@@ -345,6 +345,41 @@ def test_qtts_backbone_prefill(lib, model):
     assert fn(_ptr(ws), wsb, _ptr(table), 2, _ptr(norm), _ptr(cos), _ptr(sin), _ptr(kc), _ptr(vc), max_seq, 0, 0,
               None, _ptr(xd), _ptr(hid), None, 0, None, None, 0, -1, 0, None, 0, _stream()) != 0
     assert lib.qtts_prefill_workspace_bytes(0, 0) == 0
+
+
+class Sampling(ctypes.Structure):
+    _fields_ = [("do_sample", I), ("temperature", F), ("top_k", I), ("top_p", F), ("seed", ctypes.c_ulonglong)]
+
+
+@pytest.mark.parametrize("top_k,top_p", [(1, 1.0), (50, 1.0), (64, 0.6), (300, 1.0), (0, 0.8)])
+@pytest.mark.parametrize("temperature", [0.7, -0.7, -4.0])
+def test_prefill_selection_at_either_sign_of_temperature(lib, model, temperature, top_k, top_p):
+    """The C entries take any temperature, and a negative one reverses the order of the scaled logits: top-k,
+    top-p and the draw go by logits / temperature as the oracle computes it (no masked ids here)."""
+    sd, tw = model
+    layers = [[t.cuda().contiguous() for t in tw.bb_layers[0]]]
+    table, norm, head = _layer_table(layers), tw.bb_norm.cuda(), tw.codec_head.cuda()
+    max_seq, vocab = 16, 3072
+    cos, sin = (t.cuda() for t in rope_tables(max_seq, 128, 1e6))
+    lib.qtts_prefill_workspace_bytes.argtypes = [I, I]
+    lib.qtts_prefill_workspace_bytes.restype = ctypes.c_size_t
+    wsb = lib.qtts_prefill_workspace_bytes(1, vocab)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    fn = lib.qtts_backbone_prefill
+    fn.argtypes = [P, ctypes.c_size_t, P, I, P, P, P, P, P, I, I, I, P, P, P, P, I, P, P, I, I, I, P, I, P]
+    fn.restype = I
+    kc = torch.zeros(1, 8, max_seq, 128, dtype=torch.bfloat16, device="cuda")
+    vc, hid = torch.zeros_like(kc), torch.empty(1024, device="cuda")
+    x = torch.randn(1, 1024, generator=torch.Generator().manual_seed(12)).to(torch.bfloat16).cuda()
+    logits, tok = torch.empty(vocab, device="cuda"), torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    for seed in (1, 2, 3):
+        sp = Sampling(1, temperature, top_k, top_p, seed)
+        print(f"prefill selection, temperature {temperature}, top_k {top_k}, top_p {top_p}, seed {seed}", flush=True)
+        assert fn(_ptr(ws), wsb, _ptr(table), 1, _ptr(norm), _ptr(cos), _ptr(sin), _ptr(kc), _ptr(vc), max_seq, 0, 1, None,
+                  _ptr(x), _ptr(hid), _ptr(head), vocab, _ptr(logits), _ptr(tok), 0, -1, 0, ctypes.byref(sp), 9,
+                  _stream()) == 0
+        want = sample_token(logits.cpu(), True, sp.temperature, top_k, top_p, None, seed=seed, frame_step=9, group=0)
+        assert int(tok) == want, (temperature, top_k, top_p, seed)
 
 
 def _bb_step_args(b, table, norm, cos, sin, max_seq, pos):
