@@ -1154,10 +1154,19 @@ void launch_tile(TileArgs& g, hipStream_t st) {
 //   O, D  16 x 32 up to 128, 32 x 32 to 256 (+2 to 3 either way), 32 x 64 to 512, 64 x 64 to 1024, then
 //         128 x 64; two or four waves share a block's K range where one wave's chain of MFMAs and LDS reads
 //         is what a stage waits for (0.7 to 2 us less each)
+// Past 2048 tokens those tiles no longer fit the CUs at once and the last of 288 workgroups takes as long as the
+// first 256. Tiles of four waves and at most 80 KB of LDS, two workgroups a CU, leave less of a last round (us,
+// large tile against these; they are as fast as the large ones where the count of both comes out even):
+//   QKV   128 x 128 to 4096: 2049 tokens 44.3 : 41.7, 2560 49.5 : 43.9, 3073 54.8 : 53.4, 4096 60.1 : 58.3
+//         (6000 81.2 : 86.1)
+//   GU    128 x 128 to 2688 (two rounds of 512): 2049 46.4 : 41.3, 2560 55.0 : 46.3 (3072 56.5 : 58.9)
+//   O, D  128 x 64, no K shares: O 2049 33.2 : 24.6, 3072 36.8 : 32.0, 6000 74.6 : 65.3; down 43.6 : 35.4,
+//         49.6 : 43.8, 100.4 : 92.1
 void project_qkv(TileArgs& g, hipStream_t st) {
   if (g.M <= 256) launch_tile<P_QKV, 32, 128, 1, 4, 1, 6, 64>(g, st);
   else if (g.M <= 512) launch_tile<P_QKV, 64, 128, 2, 2, 1, 5, 64>(g, st);
   else if (g.M <= 1024) launch_tile<P_QKV, 128, 128, 4, 2, 1, 4, 64>(g, st);
+  else if (g.M > 2048 && g.M <= 4096) launch_tile<P_QKV, 128, 128, 2, 2, 1, 2, 64>(g, st);
   else launch_tile<P_QKV, 256, 128, 4, 2, 1, 3, 64>(g, st);
 }
 void project_gate_up(TileArgs& g, hipStream_t st) {
@@ -1166,6 +1175,7 @@ void project_gate_up(TileArgs& g, hipStream_t st) {
   else if (g.M <= 256) launch_tile<P_GU, 64, 96, 2, 2, 1, 3, 64>(g, st);
   else if (g.M <= 512) launch_tile<P_GU, 64, 192, 2, 2, 1, 4, 64>(g, st);
   else if (g.M <= 1024) launch_tile<P_GU, 128, 192, 4, 2, 1, 3, 64>(g, st);
+  else if (g.M > 2048 && g.M <= 2688) launch_tile<P_GU, 128, 128, 2, 2, 1, 2, 64>(g, st);
   else launch_tile<P_GU, 256, 192, 4, 2, 1, 2, 64>(g, st);
 }
 // O or down: also leaves in g.nsq how many sum-of-squares parts it wrote per token
@@ -1176,7 +1186,8 @@ void project_residual(TileArgs& g, hipStream_t st) {
   else if (g.M <= 256) launch_tile<MODE, 32, 32, 2, 2, 2, 6, 128>(g, st);
   else if (g.M <= 512) launch_tile<MODE, 32, 64, 2, 2, 2, 5, 128>(g, st);
   else if (g.M <= 1024) launch_tile<MODE, 64, 64, 2, 2, 2, 4, 128>(g, st);
-  else launch_tile<MODE, 128, 64, 2, 2, 2, 3, 128>(g, st);
+  else if (g.M <= 2048) launch_tile<MODE, 128, 64, 2, 2, 2, 3, 128>(g, st);
+  else launch_tile<MODE, 128, 64, 2, 2, 1, 3, 64>(g, st);
 }
 
 

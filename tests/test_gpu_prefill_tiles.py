@@ -12,7 +12,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-2
-LAYERS = 2
+LAYERS, MAX_SEQ = 2, 4224
 
 
 def _norm(x, g):
@@ -46,13 +46,14 @@ def _reference(sd, x, cos, sin, past_k, past_v):
 @pytest.fixture(scope="module")
 def model(pkg):
     sd = pkg.synthetic_state_dict(seed=31, cfg=pkg.SyntheticConfig(n_bb_layers=LAYERS, n_cp_layers=0, n_groups=0), device="cuda")
-    return sd, pkg.TTSMegakernelGenerator(model=sd, max_seq_len=4096)
+    return sd, pkg.TTSMegakernelGenerator(model=sd, max_seq_len=MAX_SEQ)
 
 
 @pytest.mark.parametrize("tokens,prefix,distinct", [
     (1, 0, False), (15, 0, False), (16, 3, True), (17, 0, False), (32, 0, False), (33, 31, True), (128, 0, False), (129, 0, True),
     (256, 32, False), (257, 0, False), (512, 0, False), (513, 700, True), (736, 0, False), (737, 0, False), (737, 1000, True),
-    (1024, 0, False), (1025, 0, False), (1760, 0, False), (1761, 300, True), (2049, 0, False)])
+    (1024, 0, False), (1025, 0, False), (1760, 0, False), (1761, 300, True), (2048, 0, False), (2049, 0, False),
+    (2688, 0, False), (2689, 5, True), (4096, 0, False), (4097, 0, False)])
 def test_prefill_at_tile_edges(model, tokens, prefix, distinct):
     sd, bb = model
     g = torch.Generator(device="cuda").manual_seed(tokens + prefix)
@@ -83,6 +84,6 @@ def test_prefill_at_tile_edges(model, tokens, prefix, distinct):
         rows_norm = lambda t: t.square().sum(dim=(0, 1, 3)).sqrt()
         worst = float((rows_norm(a.double() - b) / rows_norm(b)).max())
         assert worst < 3 * TOL, (name, worst)
-    assert float(bb.get_k_cache()[:, :, end:].abs().max() if end < 4096 else 0) == 0.0   # nothing past the prompt
+    assert float(bb.get_k_cache()[:, :, end:].abs().max() if end < MAX_SEQ else 0) == 0.0   # nothing past the prompt
     if prefix:
         assert torch.equal(bb.get_k_cache()[:, :, :prefix], pk) and torch.equal(bb.get_v_cache()[:, :, :prefix], pv)
