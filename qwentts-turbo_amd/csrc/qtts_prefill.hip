@@ -1204,8 +1204,7 @@ Layout layout(int S, int vocab) {
   L.h = take((size_t)S * HID * 2);
   L.xg = take((size_t)S * HID * 2);
   L.ssq = take((size_t)S * SQP * 4);
-  // (the size query's lower bound counts a whole q | k | v row per token; K and V go to the cache directly)
-  L.q = take((size_t)S * (QW + 2 * NKVH * HDIM) * 2);
+  L.q = take((size_t)S * QW * 2);
   L.att = take((size_t)S * QW * 2);
   L.act = take((size_t)S * INTER * 2);
   L.logits = take((size_t)(vocab > 0 ? vocab : MAXV) * 2);

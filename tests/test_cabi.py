@@ -44,19 +44,23 @@ def test_workspace_bytes_is_callable_without_a_gpu():
 
 def test_prefill_workspace_bytes_without_a_gpu():
     """qtts_prefill_workspace_bytes is a host-only size query: 0 for an empty prompt or an
-    out-of-range vocabulary; otherwise at least the bf16 activations of every prompt row
-    (hidden, normed, q|k|v, attention, SwiGLU: 1024 + 1024 + 4096 + 2048 + 3072 per row) plus the
-    head logits. Not monotone in the prompt length (the split-K factor, and so the partials
-    buffer, changes with the row count)."""
+    out-of-range vocabulary; otherwise the activations of every prompt row (residual, normed, rotated
+    queries, attention and SwiGLU in bf16: 1024 + 1024 + 2048 + 2048 + 3072 values; 32 f32 parts of its
+    sum of squares) plus the head logits, each buffer rounded up to 256 bytes. It grows with the prompt
+    and stays below 22,528 bytes a row and 57,344 more, for which callers may have sized a workspace
+    that they keep (the size for a prompt of 4,096 tokens and more when K and V had rows of it)."""
     lib = ctypes.CDLL(str(LIB))
     f = lib.qtts_prefill_workspace_bytes
     f.restype = ctypes.c_size_t
     f.argtypes = [ctypes.c_int, ctypes.c_int]
     assert f(0, 0) == 0 and f(-1, 0) == 0 and f(128, -1) == 0 and f(128, 3073) == 0
-    for n in (1, 7, 40, 127, 128, 129, 255, 256, 333, 511, 512, 1100, 2048, 4096):
-        lower = n * (1024 + 1024 + 4096 + 2048 + 3072) * 2 + 3072 * 2
-        assert f(n, 0) >= lower, n
+    last = 0
+    for n in (1, 7, 40, 127, 128, 129, 255, 256, 333, 511, 512, 1100, 2048, 3969, 4096, 8192, 30000):
+        lower = n * ((1024 + 1024 + 2048 + 2048 + 3072) * 2 + 32 * 4) + 3072 * 2
+        assert lower <= f(n, 0) <= lower + 7 * 256, n
+        assert last < f(n, 0) <= 22528 * n + 57344, n
         assert f(n, 3072) >= f(n, 0), n
+        last = f(n, 0)
 
 
 def test_torch_extension_exposes_reference_classes(pkg):
