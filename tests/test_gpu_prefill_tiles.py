@@ -84,6 +84,32 @@ def test_prefill_at_tile_edges(model, tokens, prefix, distinct):
         rows_norm = lambda t: t.square().sum(dim=(0, 1, 3)).sqrt()
         worst = float((rows_norm(a.double() - b) / rows_norm(b)).max())
         assert worst < 3 * TOL, (name, worst)
-    assert float(bb.get_k_cache()[:, :, end:].abs().max() if end < MAX_SEQ else 0) == 0.0   # nothing past the prompt
+    for cache in (bb.get_k_cache(), bb.get_v_cache()):                          # nothing past the prompt
+        assert float(cache[:, :, end:].abs().max() if end < MAX_SEQ else 0) == 0.0
     if prefix:
         assert torch.equal(bb.get_k_cache()[:, :, :prefix], pk) and torch.equal(bb.get_v_cache()[:, :, :prefix], pv)
+
+
+@pytest.mark.parametrize("tokens,prefix", [(1, 0), (13, 20), (45, 0), (333, 7), (1000, 100), (1777, 0), (1790, 333)])
+def test_prefill_does_not_read_past_the_prompt(model, tokens, prefix):
+    """The cache rows past the prompt hold NaN: a score or a weight that took one of them (the attention reads
+    whole blocks of 32 keys) would show, also where its weight is zero. They hold it still afterwards."""
+    sd, bb = model
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    x, pk, pv = rnd(tokens, 1024), rnd(LAYERS, 8, prefix, 128), rnd(LAYERS, 8, prefix, 128)
+    end, outs = prefix + tokens, []
+    print(f"prefill over a poisoned cache: {tokens} tokens after {prefix}", flush=True)
+    for fill in (0.0, float("nan")):
+        bb.reset()
+        if prefix:
+            bb.set_kv_cache(pk, pv)
+            bb.set_position(prefix)
+        for cache in (bb.get_k_cache(), bb.get_v_cache()):
+            cache[:, :, prefix:] = fill
+        hidden = bb.prefill(x)
+        outs.append((hidden, bb.get_k_cache()[:, :, :end].clone(), bb.get_v_cache()[:, :, :end].clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    assert bool(bb.get_k_cache()[:, :, end:].isnan().all()) and bool(bb.get_v_cache()[:, :, end:].isnan().all())
+    for cache in (bb.get_k_cache(), bb.get_v_cache()):
+        cache.zero_()
