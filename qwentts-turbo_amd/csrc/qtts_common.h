@@ -363,12 +363,23 @@ __device__ __forceinline__ void philox4x64_10(uint64_t c[4], uint64_t k0, uint64
     c[0] = n0; c[1] = lo1; c[2] = n2; c[3] = lo0;
   }
 }
-__device__ __forceinline__ double sampler_uniform(uint64_t seed, int frame_step, int group, int vid) {
-  uint64_t c[4] = {(uint64_t)(vid >> 2), (uint64_t)(uint32_t)frame_step, (uint64_t)(uint32_t)group, 0ull};
+// the four words of the block of ids vid & ~3 .. vid | 3
+__device__ __forceinline__ void sampler_block(uint64_t c[4], uint64_t seed, int frame_step, int group, int vid) {
+  c[0] = (uint64_t)(vid >> 2);
+  c[1] = (uint64_t)(uint32_t)frame_step;
+  c[2] = (uint64_t)(uint32_t)group;
+  c[3] = 0ull;
   philox4x64_10(c, seed, 0x5154545341464D50ull);
+}
+__device__ __forceinline__ double sampler_word(const uint64_t c[4], int vid) {
   // selects: an indexed read would put the words in memory
   const uint64_t lo = (vid & 1) ? c[1] : c[0], hi = (vid & 1) ? c[3] : c[2];
   return ((double)(((vid & 2) ? hi : lo) >> 12) + 0.5) * (1.0 / 4503599627370496.0);
+}
+__device__ __forceinline__ double sampler_uniform(uint64_t seed, int frame_step, int group, int vid) {
+  uint64_t c[4];
+  sampler_block(c, seed, frame_step, group, vid);
+  return sampler_word(c, vid);
 }
 
 // Order-preserving map float -> uint32 (larger float, larger key).

@@ -1471,7 +1471,7 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
 
   if (poller) {
     int npass = 0;   // layer passes begun
-    walk([&](int st, int pi, int layer) {
+    walk([&](int st, int pi, int layer) QTTS_INLINE {
       lane = opaque(lane);
       if (st == S_QKV || st == S_QKV2) {
         if (npass > 0) P.ec.spin_cap = a.spin_cap;
@@ -1635,7 +1635,7 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
       }
     });
   } else {
-    walk([&](int st, int pi, int layer) {
+    walk([&](int st, int pi, int layer) QTTS_INLINE {
       lane = opaque(lane);
       const PosInfo q = pinfo(pi);
       const int lp = pi * NL + layer;

@@ -26,12 +26,12 @@ __device__ __forceinline__ void best_merge(float& bv, int& bi, float ov, int oi)
 }
 
 // LDS scratch of one selection: the short list (and a slot per lane for the writes that it does not
-// take); when more than SEL_CAP ids stay in the running, every logit and its probability (top-p).
+// take); for draws in place, every logit by id and its probability (top-p).
 // Entries are words key << 16 | id.
 constexpr int SEL_CAP = 256;
 struct SelScratch {
   uint32_t list[SEL_CAP + 64];
-  uint32_t all[MAXV];
+  alignas(16) uint32_t all[MAXV];
   double p[MAXV];
 };
 
@@ -99,9 +99,11 @@ __device__ __forceinline__ int greedy_id(uint32_t best, int n) {
 // k-th largest of the 64 lane maxima is a lower bound of the k-th largest logit: about 90 of 2048 ids
 // reach it and go to a short list of at most SEL_CAP, and the temperature division, the exact threshold,
 // the Philox draws (one pass of 64 lanes for 64 ids) and the logarithms run on that list alone. A larger
-// top_k, or ties that overflow the list, search the threshold on the registers; more than SEL_CAP kept ids
-// are drawn in place. A threshold search over 32-bit keys in LDS and a draw in every lane pass that held a
-// kept id took 93 us for a code-predictor head of 2048 (top-k 50), 15 of them a frame.
+// top_k, or ties that overflow the list, search the threshold on the registers. No top_k, or one past SEL_CAP
+// ids, draws in place, the words in LDS by id so that four neighbours share a Philox block (without: a frame
+// of unlimited draws took 1,576 us, now 1,355, and 8 of them 2,112, now 1,902). A threshold search over 32-bit
+// keys in LDS and a draw in every lane pass that held a kept id took 93 us for a code-predictor head of 2048
+// (top-k 50), 15 of them a frame.
 constexpr int SEL_NJ = MAXV / 64;          // words per lane
 __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, const SelParams& sp, SelScratch* sc) {
   const int lane = opaque((int)threadIdx.x & 63);
@@ -202,7 +204,14 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
 
   const bool limited = sp.top_k > 0 && sp.top_k < n;
   const bool reversed = __builtin_signbit(T);   // the scaled values fall as the keys rise: everything on scaled words
-  int n_in = -1;                           // words to draw from, in the list or (more than SEL_CAP) in `all`
+  int n_in = -1;                           // words to draw from in the list
+  double best = -INFINITY;
+  int bi = 0x7fffffff;
+  auto draw = [&](uint32_t e, double u) QTTS_SEL_INLINE {
+    const int id = (int)(e & 0xffffu);
+    const double g = (double)bfkey_value(e >> 16) - log(-log(u));
+    if (g > best || (g == best && id < bi)) { best = g; bi = id; }
+  };
   if (limited && sp.top_k <= 64 && !reversed) {
     uint32_t lmax[1] = {0u};
 #pragma unroll
@@ -231,15 +240,18 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
     // a NaN that is kept makes the mass under top-p no number, also one with its sign bit set (below -inf)
     const bool no_mass = !reversed && sp.top_p < 1.0f && thr < SEL_NINF && (thr == 0u ? n : count(thr)) > count(SEL_NINF);
     thr = max(thr, reversed ? 0u : SEL_NINF + 1u);   // suppressed ids are never drawn
-    const int c = reversed ? SEL_CAP + 1 : (no_mass ? 0 : collect(thr));
+    const int c = no_mass ? 0 : (limited && sp.top_k <= SEL_CAP && !reversed ? collect(thr) : SEL_CAP + 1);
     if (c <= SEL_CAP) {
       n_in = finish_list(c, 0);
     } else {
-      // every scaled word in LDS (0: not kept), so that the loops below stay rolled
+      // every scaled word in LDS by its id (0: not kept), so that the loops below stay rolled
+      sc->all[0] = 0u;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) sc->all[lane + 64 * j] = w[j];
+      for (int j = 0; j < NJ; ++j)
+        if (w[j] != 0u) sc->all[w[j] & 0xffffu] = w[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll 1
-      for (int i = lane; i < MAXV; i += 64) {
+      for (int i = lane; i < n; i += 64) {
         const uint32_t e = sc->all[i];
         const float v = sel_scaled(e >> 16, T);
         sc->all[i] = e != 0u && e >= (thr << 16) && v != -INFINITY ? (bfkey(v) << 16) | (e & 0xffffu) : 0u;
@@ -251,22 +263,22 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
           const uint32_t cand = k | (1u << b);
           int kept = 0;
 #pragma unroll 1
-          for (int i = lane; i < MAXV; i += 64) kept += __popcll(__ballot(sc->all[i] >= (cand << 16)));
+          for (int i = lane; i < n; i += 64) kept += __popcll(__ballot(sc->all[i] >= (cand << 16)));
           if (kept >= sp.top_k) k = cand;
         }
 #pragma unroll 1
-        for (int i = lane; i < MAXV; i += 64)
+        for (int i = lane; i < n; i += 64)
           if (sc->all[i] < (k << 16)) sc->all[i] = 0u;
       }
-      n_in = MAXV;
+      n_in = 0;
       if (sp.top_p < 1.0f) {
         float m = -INFINITY;
-        for (int i = lane; i < MAXV; i += 64)
+        for (int i = lane; i < n; i += 64)
           if (sc->all[i] != 0u) m = fmaxf(m, bfkey_value(sc->all[i] >> 16));
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
         double z = 0.0;
-        for (int i = lane; i < MAXV; i += 64) {
+        for (int i = lane; i < n; i += 64) {
           const double pi = sc->all[i] != 0u ? exp((double)bfkey_value(sc->all[i] >> 16) - (double)m) : 0.0;
           sc->p[i] = pi;
           z += pi;
@@ -274,24 +286,31 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
         z = wave_sum_d(z);
         const uint32_t pth = top_p_key(z, [&](uint32_t t) QTTS_SEL_INLINE {
           double acc = 0.0;
-          for (int i = lane; i < MAXV; i += 64) acc += (sc->all[i] >> 16) > t ? sc->p[i] : 0.0;
+          for (int i = lane; i < n; i += 64) acc += (sc->all[i] >> 16) > t ? sc->p[i] : 0.0;
           return wave_sum_d(acc);
         });
-        for (int i = lane; i < MAXV; i += 64)
+        for (int i = lane; i < n; i += 64)
           if ((sc->all[i] >> 16) < pth) sc->all[i] = 0u;
+      }
+      // (four neighbouring ids share a Philox block)
+#pragma unroll 1
+      for (int i = 4 * lane; i < n; i += 256) {
+        const u32x4 e4 = *reinterpret_cast<const u32x4*>(&sc->all[i]);
+        if ((e4.x | e4.y | e4.z | e4.w) == 0u) continue;
+        uint64_t c[4];
+        sampler_block(c, sp.seed, sp.frame_step, sp.group, i);
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t e = sc->all[i + q];
+          if (e != 0u) draw(e, sampler_word(c, q));
+        }
       }
     }
   }
-  double best = -INFINITY;
-  int bi = 0x7fffffff;
-  const uint32_t* from = n_in <= SEL_CAP ? sc->list : sc->all;
 #pragma unroll 1
   for (int i = lane; i < n_in; i += 64) {
-    const uint32_t e = from[i];
-    if (e == 0u) continue;
-    const int id = (int)(e & 0xffffu);
-    const double g = (double)bfkey_value(e >> 16) - log(-log(sampler_uniform(sp.seed, sp.frame_step, sp.group, id)));
-    if (g > best || (g == best && id < bi)) { best = g; bi = id; }
+    const uint32_t e = sc->list[i];
+    draw(e, sampler_uniform(sp.seed, sp.frame_step, sp.group, (int)(e & 0xffffu)));
   }
   auto merge = [&](double ov, int oi) QTTS_SEL_INLINE {
     if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }

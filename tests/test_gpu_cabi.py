@@ -352,14 +352,14 @@ class Sampling(ctypes.Structure):
 
 
 @pytest.mark.parametrize("top_k,top_p", [(1, 1.0), (50, 1.0), (64, 0.6), (300, 1.0), (0, 0.8)])
-@pytest.mark.parametrize("temperature", [0.7, -0.7, -4.0])
-def test_prefill_selection_at_either_sign_of_temperature(lib, model, temperature, top_k, top_p):
+@pytest.mark.parametrize("temperature,vocab", [(0.7, 3072), (0.7, 1408), (-0.7, 3072), (-0.7, 128), (-4.0, 1408)])
+def test_prefill_selection_at_either_sign_of_temperature(lib, model, temperature, vocab, top_k, top_p):
     """The C entries take any temperature, and a negative one reverses the order of the scaled logits: top-k,
     top-p and the draw go by logits / temperature as the oracle computes it (no masked ids here)."""
     sd, tw = model
     layers = [[t.cuda().contiguous() for t in tw.bb_layers[0]]]
-    table, norm, head = _layer_table(layers), tw.bb_norm.cuda(), tw.codec_head.cuda()
-    max_seq, vocab = 16, 3072
+    table, norm, head = _layer_table(layers), tw.bb_norm.cuda(), tw.codec_head.cuda()[:vocab].contiguous()
+    max_seq = 16
     cos, sin = (t.cuda() for t in rope_tables(max_seq, 128, 1e6))
     lib.qtts_prefill_workspace_bytes.argtypes = [I, I]
     lib.qtts_prefill_workspace_bytes.restype = ctypes.c_size_t
