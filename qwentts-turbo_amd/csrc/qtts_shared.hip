@@ -218,6 +218,46 @@ __device__ __forceinline__ bool poll_sum8s(const Poll& P, const uint64_t* p0, ui
   return ok;
 }
 
+// The backbone's token selection over a stream's logit slots, kept out of line: inlined, its registers and the
+// loop-invariant parts of its sampler change the allocation of the whole launch (8 streams at 512 positions, us
+// inlined : called: greedy 796.7 : 793.1, sampled 797.4 : 793.0; the sampled instantiation's spills 4 : 0). In the
+// code predictor's frame a call for each of 15 heads costs what it saves (sampled 1,536 : 1,545). The
+// arguments are uniform and come in registers one by one (a struct of them would go through scratch memory), the
+// LDS pointers as LDS addresses.
+template <typename T>
+__device__ __forceinline__ T uni(T v) {
+  uint32_t w[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (uint32_t& x : w) x = (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ T* lds_ptr(uint32_t at) {
+  return (T*)(__attribute__((address_space(3))) T*)at;
+}
+template <bool SEL>
+__device__ __attribute__((noinline)) int sh_select(SWorkspace* ws_, uint32_t spin_cap, uint32_t off, uint32_t tag, int n,
+                                                   uint32_t pen_bits, int tail, int eos, int drop, float penalty,
+                                                   uint32_t scratch, float temperature, int top_k, float top_p, uint64_t seed,
+                                                   int frame_step) {
+  SWorkspace* ws = uni(ws_);
+  Poll P;
+  P.base = ws;
+  P.rs = __builtin_amdgcn_make_buffer_rsrc(ws, (short)0, (int)sizeof(SWorkspace), 0x00020000);
+  P.ec.err = &ws->err;
+  P.ec.spin_cap = uni(spin_cap);
+  n = uni(n);
+  const HeadMask hm = {uni(tail), uni(eos), uni(drop), uni(penalty)};
+  const uint32_t* pen = lds_ptr<uint32_t>(uni(pen_bits));
+  if constexpr (SEL) {
+    const SelParams sp = {1, uni(temperature), uni(top_k), uni(top_p), uni(seed), uni(frame_step), 0};
+    return head_sample<true>(P, uni(off), n, uni(tag), sp, hm, pen, lds_ptr<SelScratch>(uni(scratch)));
+  } else {
+    return head_argmax<true>(P, uni(off), n, uni(tag), hm, pen);
+  }
+}
 
 template <bool BB, bool SEL>
 __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
@@ -1183,9 +1223,6 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
   // only: the selection scratch overlays the projection inputs)
   auto select_full = [&](int pi) -> int {
     const int n = cp ? a.cp_vocab : a.vocab;
-    SelParams sp = a.sel;
-    sp.seed = IO->seed;
-    sp.group = cp ? pi : 0;   // CP head pi-1 selects codebook group pi
     HeadMask hm = {n, -1, -1, 1.0f};
     if (!cp) {
       // suppress ids [V-1024, V) except EOS (generator.py:71-75)
@@ -1205,8 +1242,16 @@ __global__ void __launch_bounds__(STHR, 1) qtts_shared_kernel(const SArgs a) {
       }
     }
     const uint32_t off = ws_off(P, &ws->logits[pi & 1][wv][0]), tag = a.tag_base + TAG_HEAD + (uint32_t)pi;
-    if constexpr (SEL) return head_sample<BB>(P, off, n, tag, sp, hm, s.pen_bits[wv], &s.sel);
-    else return head_argmax<BB>(P, off, n, tag, hm, s.pen_bits[wv]);
+    SelParams sp = a.sel;
+    sp.seed = IO->seed;
+    sp.group = cp ? pi : 0;   // CP head pi-1 selects codebook group pi
+    if constexpr (BB) {
+      const auto lds_at = [](auto* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)p; };
+      return uni(sh_select<SEL>(ws, P.ec.spin_cap, off, tag, n, lds_at(s.pen_bits[wv]), hm.tail, hm.eos, hm.drop, hm.penalty,
+                                lds_at(&s.sel), sp.temperature, sp.top_k, sp.top_p, sp.seed, sp.frame_step));
+    } else {
+      return head_sample<false>(P, off, n, tag, sp, hm, s.pen_bits[wv], &s.sel);
+    }
   };
 
   // =========================================================================================
