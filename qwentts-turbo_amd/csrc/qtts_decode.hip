@@ -1471,7 +1471,7 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
 
   if (poller) {
     int npass = 0;   // layer passes begun
-    walk([&](int st, int pi, int layer) QTTS_INLINE {
+    auto step = [&](int st, int pi, int layer) {
       lane = opaque(lane);
       if (st == S_QKV || st == S_QKV2) {
         if (npass > 0) P.ec.spin_cap = a.spin_cap;
@@ -1633,9 +1633,12 @@ __global__ void __launch_bounds__(NTHR, 1) qtts_decode_kernel(const KArgs a) {
           }
           break;
       }
-    });
+    };
+    // (the sampled launches' step is too large to be inlined by itself; forced in the greedy ones it moves registers)
+    if constexpr (SEL) walk([&](int st, int pi, int layer) QTTS_INLINE { [[clang::always_inline]] step(st, pi, layer); });
+    else walk(step);
   } else {
-    walk([&](int st, int pi, int layer) QTTS_INLINE {
+    walk([&](int st, int pi, int layer) {
       lane = opaque(lane);
       const PosInfo q = pinfo(pi);
       const int lp = pi * NL + layer;
