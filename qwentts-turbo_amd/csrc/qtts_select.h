@@ -95,16 +95,20 @@ __device__ __forceinline__ int greedy_id(uint32_t best, int n) {
 // value's). Returns the same id on every lane.
 //
 // One wave at a time can issue about one instruction per 4 cycles, so the work is kept to a few
-// instructions per logit and the expensive parts to the ids still in the running. For top_k <= 64 the
-// k-th largest of the 64 lane maxima is a lower bound of the k-th largest logit: about 90 of 2048 ids
-// reach it and go to a short list of at most SEL_CAP, and the temperature division, the exact threshold,
-// the Philox draws (one pass of 64 lanes for 64 ids) and the logarithms run on that list alone. A larger
-// top_k, or ties that overflow the list, search the threshold on the registers. No top_k, or one past SEL_CAP
-// ids, draws in place, the words in LDS by id so that four neighbours share a Philox block (without: a frame
-// of unlimited draws took 1,576 us, now 1,355, and 8 of them 2,112, now 1,902). A threshold search over 32-bit
-// keys in LDS and a draw in every lane pass that held a kept id took 93 us for a code-predictor head of 2048
-// (top-k 50), 15 of them a frame.
+// instructions per logit and the expensive parts to the ids still in the running. For top_k <= 63 the
+// k-th largest of the 64 lane maxima is a lower bound of the k-th largest logit: the ids that reach it (94 of
+// 2048 on average at 50, 164 at 60, 228 at 63, where 256 is passed in a quarter of the draws) go to a short
+// list of at most SEL_CAP, and the temperature division, the exact threshold, the Philox draws (one pass of 64
+// lanes for 64 ids) and the logarithms run on that list alone. A larger top_k, or ties that overflow the list,
+// search the threshold on the registers. No top_k, or one past SEL_CAP ids, draws in place, the words in LDS by
+// id so that four neighbours share a Philox block (a frame of unlimited draws 1,577 -> 1,347 us, 8 of them
+// 2,115 -> 1,907). A threshold search over 32-bit keys in LDS and a draw in every lane pass that held a kept id
+// took 93 us for a code-predictor head of 2048 (top-k 50), 15 of them a frame.
 constexpr int SEL_NJ = MAXV / 64;          // words per lane
+// Largest top_k for the list. At 64 the bound is the smallest lane maximum, more than half of the lists overflow
+// and are searched again (us, list : search: 63 a frame 1,031 : 1,071, a backbone step 482 : 490, 8 frames
+// 1,657 : 1,653; 64 1,072 : 1,064, 492 : 490, 1,683 : 1,648)
+constexpr int SEL_LIST_K = 63;
 __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, const SelParams& sp, SelScratch* sc) {
   const int lane = opaque((int)threadIdx.x & 63);
   const float T = sp.temperature;
@@ -212,7 +216,7 @@ __device__ __forceinline__ int wave_sample(const uint32_t (&w)[SEL_NJ], int n, c
     const double g = (double)bfkey_value(e >> 16) - log(-log(u));
     if (g > best || (g == best && id < bi)) { best = g; bi = id; }
   };
-  if (limited && sp.top_k <= 64 && !reversed) {
+  if (limited && sp.top_k <= SEL_LIST_K && !reversed) {
     uint32_t lmax[1] = {0u};
 #pragma unroll
     for (int j = 0; j < NJ; ++j) lmax[0] = max(lmax[0], w[j]);

@@ -1,8 +1,10 @@
 """Token selection (temperature, top-k, top-p, Gumbel-max) against the oracle's sampler on the GPU's own
-logits: every branch of ``wave_select``. top_k up to 64 takes the short list from the lane maxima, larger
-ones the search over all keys, more than 256 kept ids (or no top-k) are drawn in place; rows repeated in the
-head make hundreds of exact ties, which top-k keeps; temperatures apart from 1 let neighbouring bf16 logits
-fall together. The id is exact: the same filter on the same bf16 logits and the same noise in f64.
+logits, through the prefill and the batch-1 backbone step: ``wave_sample``'s short list from the lane maxima
+(top_k up to 63), its search over all keys (larger ones) and its draws in place (more than 256 kept ids, or no
+top-k); rows repeated in the head make hundreds of exact ties, which top-k keeps; temperatures apart from 1 let
+neighbouring bf16 logits fall together. The id is exact: the same filter on the same bf16 logits and the same
+noise in f64. The other entry points, infinite and NaN logits, extreme temperatures, masks and penalties are in
+test_gpu_select_paths.py.
 """
 import pytest
 import torch
@@ -24,7 +26,7 @@ def base(pkg):
 
 
 @pytest.mark.parametrize("head", list(HEADS))
-@pytest.mark.parametrize("top_k,top_p", [(1, 1.0), (2, 1.0), (50, 1.0), (64, 1.0), (65, 1.0), (200, 1.0), (256, 1.0),
+@pytest.mark.parametrize("top_k,top_p", [(1, 1.0), (2, 1.0), (50, 1.0), (63, 1.0), (64, 1.0), (65, 1.0), (200, 1.0), (256, 1.0),
                                          (300, 1.0), (2047, 1.0), (0, 1.0), (50, 0.9), (64, 0.3), (300, 0.8), (0, 0.5)])
 def test_selection_branches(pkg, base, head, top_k, top_p):
     sd = dict(base)
