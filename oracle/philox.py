@@ -5,7 +5,7 @@ TEST INFRASTRUCTURE ONLY. Nothing in the product package imports this module; it
 checker for the HIP sampler (``qtts_philox4x64`` in the device code).
 
 Why a counter-based RNG: the reference samples with ``torch.multinomial``
-(/root/reference/qwentts_turbo/generator.py:206-207), whose stream is not reproducible across
+(qwentts_turbo/generator.py:206-207), whose stream is not reproducible across
 devices, so no sampled token of the reference can be reproduced. The build defines the sampler
 as Gumbel-max over the same filtered logits (same distribution as softmax+multinomial, see
 ``oracle.qtts_oracle.sample_token``) with the noise drawn from Philox-4x64-10, so that the

@@ -6,17 +6,17 @@ product package (``qwentts-turbo_amd/``) never imports it; its decode path runs 
 kernels and raises when they are not built.
 
 What it restates (reference file:line):
-  * backbone decode step  -- /root/reference/qwentts_turbo/csrc/fused_decode_tts.cu:728-831
+  * backbone decode step  -- qwentts_turbo/csrc/fused_decode_tts.cu:728-831
     (phases :56-157 QKV+RMSNorm, :163-276 q/k-norm+RoPE+KV write, :282-385 attention,
     :391-547 O-proj/post-norm/SwiGLU/down, :796-830 final norm)
-  * code-predictor step   -- /root/reference/qwentts_turbo/csrc/fused_decode_code_predictor.cu:565-668
-  * RoPE tables           -- /root/reference/qwentts_turbo/megakernel_backbone.py:392-398,
-                             /root/reference/qwentts_turbo/megakernel_code_predictor.py:297-308
-  * interleaved 3D mRoPE  -- /root/reference/qwentts_turbo/csrc/rope_multimodal.cuh:9-54 (intent);
+  * code-predictor step   -- qwentts_turbo/csrc/fused_decode_code_predictor.cu:565-668
+  * RoPE tables           -- qwentts_turbo/megakernel_backbone.py:392-398,
+                             qwentts_turbo/megakernel_code_predictor.py:297-308
+  * interleaved 3D mRoPE  -- qwentts_turbo/csrc/rope_multimodal.cuh:9-54 (intent);
                              index map from transformers qwen3_vl ``apply_interleaved_mrope``
   * frame loop, combine, suppress mask, repetition penalty, sampling
-                          -- /root/reference/qwentts_turbo/generator.py:71-75, 77-176, 178-207,
-                             309-362; /root/reference/tests/test_audio.py:64-184
+                          -- qwentts_turbo/generator.py:71-75, 77-176, 178-207,
+                             309-362; tests/test_audio.py:64-184
 
 Precision policies (``policy=``):
   * ``"kernel"``  -- the arithmetic the HIP kernels implement: every dot product, norm and

@@ -1,6 +1,6 @@
 """qwentts-turbo for MI355X: Qwen3-TTS decode (backbone + code predictor) as persistent gfx950 kernels.
 
-Public surface mirrors the reference package (/root/reference/qwentts_turbo/__init__.py:3-4):
+Public surface mirrors the reference package (qwentts_turbo/__init__.py:3-4):
 ``NativeTTSGenerator`` plus the two kernel wrappers. Import name: ``qwentts_turbo_amd``.
 """
 from .batched import BatchedTTSDecoder

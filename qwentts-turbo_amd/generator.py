@@ -1,6 +1,6 @@
 """NativeTTSGenerator: the reference's generation loop with every per-token step on MI355X.
 
-Mirrors /root/reference/qwentts_turbo/generator.py:21-362 and keeps ``generate()``'s signature
+Mirrors qwentts_turbo/generator.py:21-362 and keeps ``generate()``'s signature
 (:77-81). What moved on-device, per codec frame:
   * the whole code-predictor loop (:309-354) -- 2-token prefill, 14 decode steps, 15 lm-heads
     with token selection and embedding gathers -- plus the 16-codebook embedding combine and

@@ -1,6 +1,6 @@
 """Backbone (talker) decode on MI355X: the reference's ``TTSMegakernelGenerator`` interface.
 
-Mirrors /root/reference/qwentts_turbo/megakernel_backbone.py:412-488 (wrapper) and :358-409
+Mirrors qwentts_turbo/megakernel_backbone.py:412-488 (wrapper) and :358-409
 (weight extraction). The kernel is the persistent gfx950 backbone kernel of
 ``csrc/qtts_decode.hip`` reached through ``_qwentts_amd_C.MegakernelTTSDecoder``.
 Differences from the reference: weights come from a state dict / module / local safetensors

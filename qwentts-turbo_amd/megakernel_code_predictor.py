@@ -1,6 +1,6 @@
 """Code-predictor decode on MI355X: the reference's ``CodePredictorMegakernelGenerator`` interface.
 
-Mirrors /root/reference/qwentts_turbo/megakernel_code_predictor.py:319-350 (wrapper) and
+Mirrors qwentts_turbo/megakernel_code_predictor.py:319-350 (wrapper) and
 :265-316 (weight extraction; RoPE theta 1e6, bf16 tables). Besides the reference's
 single-step decoder it binds the 15 lm-heads and codebook embeddings so a whole frame (the
 2-token prefill, 14 decode steps, 15 heads with on-device selection and the embedding

@@ -2,9 +2,9 @@
 
 Key names follow the Qwen3-TTS checkpoint layout the reference reads through qwen_tts
 (``talker.model.*``, ``talker.codec_head``, ``talker.code_predictor.*``; see
-/root/reference/qwentts_turbo/megakernel_backbone.py:358-409,
-/root/reference/qwentts_turbo/megakernel_code_predictor.py:265-316 and
-/root/reference/qwentts_turbo/generator.py:55-69).
+qwentts_turbo/megakernel_backbone.py:358-409,
+qwentts_turbo/megakernel_code_predictor.py:265-316 and
+qwentts_turbo/generator.py:55-69).
 """
 from __future__ import annotations
 

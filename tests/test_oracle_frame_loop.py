@@ -1,7 +1,7 @@
 """Pin the oracle's frame-loop recursion against transformers' Qwen3-Omni talker (CPU only).
 
 The code-predictor loop of one codec frame and the embedding combine are restated by the
-oracle from /root/reference/qwentts_turbo/generator.py:309-354 (2-token prefill
+oracle from qwentts_turbo/generator.py:309-354 (2-token prefill
 ``[bf16(h), emb_bb[g0]]`` at positions 0 and 1, then ``lm_head[g]`` on the last hidden and
 ``emb[g-1](token)`` as the next input) and :356-362 plus :143-149 (sum of the 16 codebook
 embeddings, then the trailing-text row of the frame or the pad row). transformers in this

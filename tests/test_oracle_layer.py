@@ -1,8 +1,8 @@
 """Pin the oracle's decoder math against transformers' Qwen3 modules (CPU only).
 
 The reference's PyTorch decode path is transformers' Qwen3 decoder layer (the talker of
-qwen_tts, run by /root/reference/qwentts_turbo/generator.py:227-243 and
-/root/reference/tests/test_audio.py:104-184). transformers is importable here, so its
+qwen_tts, run by qwentts_turbo/generator.py:227-243 and
+tests/test_audio.py:104-184). transformers is importable here, so its
 ``Qwen3Model`` -- RMSNorm, q/k-norm, rotate_half RoPE, GQA with repeat_kv, SwiGLU, eager
 attention -- is the library routine the oracle's layer is checked against:
 

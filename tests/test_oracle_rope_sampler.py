@@ -2,7 +2,7 @@
 rules (CPU only).
 
 * mRoPE: against transformers ``Qwen3VLTextRotaryEmbedding`` (its ``apply_interleaved_mrope``
-  is the index map /root/reference/qwentts_turbo/csrc/rope_multimodal.cuh:9-54 describes),
+  is the index map qwentts_turbo/csrc/rope_multimodal.cuh:9-54 describes),
   evaluated in f32 and cast to bf16, which must equal the oracle's gather from the 1D bf16
   tables bit for bit; and the reduction t == h == w -> 1D row.
 * 1D RoPE tables: against transformers ``Qwen3RotaryEmbedding`` cast to bf16.
