@@ -32,8 +32,8 @@ extern "C" {
 
 /* Per-layer weight pointers, in the reference's struct order: bf16 tensors, row-major
  * [out, in] as nn.Linear stores them.
- * Replaces: TTSLayerWeights   (/root/reference/qwentts_turbo/csrc/fused_decode_tts.cu:22-34)
- *           CPLayerWeights    (/root/reference/qwentts_turbo/csrc/fused_decode_code_predictor.cu:30-42)
+ * Replaces: TTSLayerWeights   (qwentts_turbo/csrc/fused_decode_tts.cu:22-34)
+ *           CPLayerWeights    (qwentts_turbo/csrc/fused_decode_code_predictor.cu:30-42)
  * Host mirrors: megakernel_backbone.py:43-55, megakernel_code_predictor.py:47-59. */
 typedef struct TTSLayerWeights {
     const void* input_layernorm_weight;     /* [1024]        */
@@ -67,7 +67,7 @@ typedef TTSLayerWeights CPLayerWeights;
  * < max_seq_len; attn_scale is 1/sqrt(128). cos_table / sin_table: bf16 [>= max_seq_len, 128].
  * ------------------------------------------------------------------------------------- */
 
-/* Replaces: launch_tts_decode (/root/reference/qwentts_turbo/csrc/fused_decode_tts.cu:664-722) */
+/* Replaces: launch_tts_decode (qwentts_turbo/csrc/fused_decode_tts.cu:664-722) */
 hipError_t launch_tts_decode(
     int input_token_id, const void* embed_weight, const TTSLayerWeights* layer_weights,
     const void* final_norm_weight, const void* cos_table, const void* sin_table,
@@ -76,7 +76,7 @@ hipError_t launch_tts_decode(
     void* g_normalized, int num_layers, int position, int cache_len, int max_seq_len,
     float attn_scale, hipStream_t stream);
 
-/* Replaces: launch_tts_decode_with_embedding (/root/reference/qwentts_turbo/csrc/fused_decode_tts.cu:834-890) */
+/* Replaces: launch_tts_decode_with_embedding (qwentts_turbo/csrc/fused_decode_tts.cu:834-890) */
 hipError_t launch_tts_decode_with_embedding(
     const void* input_embedding, const TTSLayerWeights* layer_weights,
     const void* final_norm_weight, const void* cos_table, const void* sin_table,
@@ -106,7 +106,7 @@ hipError_t launch_tts_decode_with_embedding_static(
     void* g_normalized, int num_layers, int position, int cache_len, int max_seq_len,
     float attn_scale, hipStream_t stream);
 
-/* Replaces: launch_cp_decode_with_embedding (/root/reference/qwentts_turbo/csrc/fused_decode_code_predictor.cu:674-730) */
+/* Replaces: launch_cp_decode_with_embedding (qwentts_turbo/csrc/fused_decode_code_predictor.cu:674-730) */
 hipError_t launch_cp_decode_with_embedding(
     const void* input_embedding, const CPLayerWeights* layer_weights,
     const void* final_norm_weight, const void* cos_table, const void* sin_table,
@@ -176,7 +176,10 @@ hipError_t qtts_debug_trace(void* device_buffer, size_t bytes);
  * Mirrors generator.py:178-207: optional EOS suppression, greedy argmax (lowest index on
  * ties) or temperature -> top-k (ties with the k-th value kept) -> top-p (a value is kept
  * when the probability mass of strictly larger values is <= top_p) -> Gumbel-max draw with
- * Philox-4x64-10 noise keyed by (seed, frame_step, group, vocab id). */
+ * Philox-4x64-10 noise keyed by (seed, frame_step, group, vocab id). A negative temperature
+ * reverses the order of the values. A NaN logit ranks above +inf (below -inf with its sign bit
+ * set) and is never taken; when nothing can be drawn (every id masked, or a mass that is NaN)
+ * the largest logit is, lowest index on ties. */
 typedef struct QttsSampling {
     int do_sample;
     float temperature;
@@ -274,8 +277,8 @@ hipError_t qtts_backbone_step_streams(
  * [num_layers, 8, max_seq_len, 128], the decode layout); attention covers cache positions
  * 0 .. position + n_tokens - 1 (causal), so a prefix already in the cache is attended.
  * Arithmetic follows the transformers bf16 forward (bf16 storage after every op, f32 sums on
- * bf16 MFMA; the layer norms' rstd scales the f32 sums of the projection after them). pos3: NULL (t = h = w = position of the token) or device int32 [3][n_tokens]
- * rotary (t, h, w) rows of the bf16 tables (clamped to [0, max_seq_len)). out_hidden: f32 [1024],
+ * bf16 MFMA; the layer norms' rstd scales the f32 sums of the projection after them). pos3: NULL
+ * (t = h = w = position of the token) or device int32 [3][n_tokens] rotary (t, h, w) rows of the bf16 tables (clamped to [0, max_seq_len)). out_hidden: f32 [1024],
  * the final-norm hidden of the last token (bf16 values). When codec_head is not NULL the first
  * group-0 token is selected from bf16(codec_head . hidden) as in generator.py:113-119 (suppress
  * mask when mask_tail, EOS removed when suppress_eos, greedy or sampled) into out_token; the

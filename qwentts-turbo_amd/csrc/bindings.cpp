@@ -1,7 +1,7 @@
 // PyTorch-ROCm extension: the reference's pybind classes over the C ABI of libqwentts_amd.
 //
-// MegakernelTTSDecoder           -- /root/reference/qwentts_turbo/megakernel_backbone.py:109-332
-// MegakernelCodePredictorDecoder -- /root/reference/qwentts_turbo/megakernel_code_predictor.py:86-242
+// MegakernelTTSDecoder           -- qwentts_turbo/megakernel_backbone.py:109-332
+// MegakernelCodePredictorDecoder -- qwentts_turbo/megakernel_code_predictor.py:86-242
 //
 // Same constructor arguments, method names and return conventions as the reference (outputs
 // are fresh tensors; KV getters alias the internal caches). Differences: shapes, dtypes,

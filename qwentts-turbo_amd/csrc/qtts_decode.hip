@@ -1,8 +1,8 @@
 // Persistent decode kernels for Qwen3-TTS on MI355X (gfx950).
 //
 // Semantics follow the reference megakernels:
-//   backbone:       /root/reference/qwentts_turbo/csrc/fused_decode_tts.cu:728-831
-//   code predictor: /root/reference/qwentts_turbo/csrc/fused_decode_code_predictor.cu:565-668
+//   backbone:       qwentts_turbo/csrc/fused_decode_tts.cu:728-831
+//   code predictor: qwentts_turbo/csrc/fused_decode_code_predictor.cu:565-668
 // with the interleaved 3D mRoPE of rope_multimodal.cuh:9-54 (t, h, w may differ) and the
 // frame glue of generator.py:116-174, 178-207, 309-362 moved on-device.
 //

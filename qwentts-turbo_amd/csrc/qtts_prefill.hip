@@ -402,25 +402,19 @@ __global__ void __launch_bounds__(64 * AW, 2) attn_kernel(const bf16_t* qrows, c
   }
 }
 
-// Wait until at most N of this wave's vector-memory instructions are in flight (the compiler does not
-// track LDS writes made by DMA).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N <= 63, "vmcnt field");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-// ... and none of its LDS reads
+// Wait until at most N of this wave's vector-memory instructions and none of its LDS reads are in flight (the
+// compiler does not track LDS writes made by DMA).
 template <int N>
 __device__ __forceinline__ void wait_vm_lds() {
   static_assert(N >= 0 && N <= 63, "vmcnt field");
   __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
 }
 
-// The same attention for long prompts, one workgroup of 8 waves per (32-query block, KV head): wave (hd, ks) takes query head 2 kvh + hd and the 32-key
-// blocks kb = ks, ks + 4, ... in one pass with a running (online) softmax. The two heads of a KV head share
-// each staged K and V block, and the queries stay in registers, so that a wave's 32 x 32 block costs 24 KB of
-// LDS traffic (40 KB in attn_kernel). 47 -> 38 us at 2048 tokens, 18.7 -> 16.8 at 1000.
+// The same attention for long prompts, one workgroup of 8 waves per (32-query block, KV head): wave (hd, ks)
+// takes query head 2 kvh + hd and the 32-key blocks kb = ks, ks + 4, ... in one pass with a running (online)
+// softmax. The two heads of a KV head share each staged K and V block, and the queries stay in registers, so
+// that a wave's 32 x 32 block costs 24 KB of LDS traffic (40 KB in attn_kernel): 44.8 -> 34.6 us at 2048 tokens
+// (kernel trace).
 // What bounds it now is the chain of a step (1.6 us: wait and barrier 0.4, copies issued 0.3, scores, softmax and
 // P V 0.3 each) at two waves a SIMD: taking the next block's scores under this one's softmax, or staging through
 // registers two steps ahead, changed nothing.
@@ -428,9 +422,8 @@ __device__ __forceinline__ void wait_vm_lds() {
 //     (16 bytes) of row r sits at position c ^ (r & 7).
 //   * The layouts of S^T, P and O^T are attn_kernel's; O^T and l are rescaled only when some query's block
 //     max passes the running one by more than 2^8.
-// The key splits of a
-// head merge through LDS in split order, wave ks finishing dims 32 ks .. 32 ks + 31. Workgroups: KV head =
-// linear id mod 8 (one head per XCD's L2), the longest query blocks first.
+// The key splits of a head merge through LDS in split order, wave ks finishing dims 32 ks .. 32 ks + 31.
+// Workgroups: KV head = linear id mod 8 (one head per XCD's L2), the longest query blocks first.
 constexpr int AKS = 4;                              // key splits
 constexpr int ABLK = 32 * HDIM * 2;                 // bytes of a K or V block
 constexpr int ATTP_SMEM = AKS * 2 * 2 * ABLK + 2 * AKS * 2 * 32 * 4;   // (K, V) x 2 buffers per split; (m, l) of the merge
@@ -626,7 +619,7 @@ __global__ void __launch_bounds__(128 * AKS, 2) attn_pair_kernel(const bf16_t* q
     L += mv == -INFINITY ? 0.0f : sml[(v * 2 + 1) * 32 + c] * __builtin_amdgcn_exp2f((mv - M) * SL);
   }
   const float sw = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * SL);
-  // part [head][split][32 dims][64 lanes]: wave ks leaves its sums of the dims that another wave finishes
+  // [head][split][dim block][register quad][lane][4]: every wave leaves its sums of all 128 dims
   float* ob = reinterpret_cast<float*>(smem) + hd * AKS * 64 * 64;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
@@ -1143,9 +1136,10 @@ void launch_tile(TileArgs& g, hipStream_t st) {
 }
 
 // Tiles by prompt length M. A projection's time is its workgroups' K loop (operand bytes per CU through
-// LDS) plus about 4 us of launch, first loads and epilogue, so the tile grows with M as slowly as 256
-// workgroups, one a CU, allow. Measured over prompts of 13 to 2048 tokens, without reads ahead (us a layer, against the best
-// alternative):
+// LDS) plus about 4 us of launch, first loads and epilogue, so the tile grows with M as slowly as one round of at
+// most 256 workgroups, one a CU, allows: it doubles at 256, 512 and 1024 tokens, where a grid is whole, and just
+// past them 144 to 192 workgroups run; up to 32 tokens QKV, O and down have 32, gate/up 96 or 192. Measured over
+// prompts of 13 to 2048 tokens, without reads ahead (us a layer, against the best alternative):
 //   QKV (a head's 128 columns)  32 tokens up to 256, 64 to 512, 128 to 1024, then 256; a step too small
 //                               or too large costs 2 to 10 us
 //   GU    16 x 64 up to 32 tokens (at 13: 1.2 us less than 32 x 96), 32 x 96 to 128, 64 x 96 to 256 (32 x 96:
@@ -1154,9 +1148,9 @@ void launch_tile(TileArgs& g, hipStream_t st) {
 //   O, D  16 x 32 up to 128, 32 x 32 to 256 (+2 to 3 either way), 32 x 64 to 512, 64 x 64 to 1024, then
 //         128 x 64; two or four waves share a block's K range where one wave's chain of MFMAs and LDS reads
 //         is what a stage waits for (0.7 to 2 us less each)
-// Past 2048 tokens those tiles no longer fit the CUs at once and the last of 288 workgroups takes as long as the
-// first 256. Tiles of four waves and at most 80 KB of LDS, two workgroups a CU, leave less of a last round (us,
-// large tile against these; they are as fast as the large ones where the count of both comes out even):
+// Past 2048 tokens those tiles no longer fit the CUs at once, and the last 32 of 288 workgroups take as long as
+// the first 256. Tiles of four waves and at most 80 KB of LDS, two workgroups a CU, leave less of a last round
+// (us, large tile : these):
 //   QKV   128 x 128 to 4096: 2049 tokens 44.3 : 41.7, 2560 49.5 : 43.9, 3073 54.8 : 53.4, 4096 60.1 : 58.3
 //         (6000 81.2 : 86.1)
 //   GU    128 x 128 to 2688 (two rounds of 512): 2049 46.4 : 41.3, 2560 55.0 : 46.3 (3072 56.5 : 58.9)
@@ -1256,8 +1250,8 @@ hipError_t qtts_backbone_prefill(void* workspace, size_t workspace_bytes, const 
   const auto* cs = static_cast<const bf16_t*>(cos_table);
   const auto* sn = static_cast<const bf16_t*>(sin_table);
   const float scale = 1.0f / sqrtf((float)HDIM);
-  const unsigned norm_grid = (unsigned)((S + 3) / 4);
-  hipLaunchKernelGGL(embed_kernel, dim3(norm_grid), dim3(256), 0, stream, static_cast<const bf16_t*>(input_embeddings),
+  const unsigned embed_grid = (unsigned)((S + 3) / 4);
+  hipLaunchKernelGGL(embed_kernel, dim3(embed_grid), dim3(256), 0, stream, static_cast<const bf16_t*>(input_embeddings),
                      layer_weights, h, xg, ssq, S);
   TileArgs g{};
   g.layers = layer_weights;

@@ -1822,8 +1822,9 @@ hipError_t qtts_backbone_step_shared(int n_streams, void* workspace, const TTSLa
     io.skip = in.skip_if;
   }
   assign_units(a);
-  return qtts_host::launch_persistent(a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<true, true> : (const void*)qtts::sh::qtts_shared_kernel<true, false>, qtts::sh::STHR, &a, &a.tag_base,
-                                      workspace, 1, sizeof(SWorkspace), stream);
+  const void* fn = a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<true, true>
+                                   : (const void*)qtts::sh::qtts_shared_kernel<true, false>;
+  return qtts_host::launch_persistent(fn, qtts::sh::STHR, &a, &a.tag_base, workspace, 1, sizeof(SWorkspace), stream);
 }
 
 hipError_t qtts_cp_frame_shared(int n_streams, void* workspace, const CPLayerWeights* layer_weights, int num_layers,
@@ -1871,8 +1872,9 @@ hipError_t qtts_cp_frame_shared(int n_streams, void* workspace, const CPLayerWei
     io.done = done + st;
     io.seed = sampling ? sampling->seed + (uint64_t)st : 0;
   }
-  return qtts_host::launch_persistent(a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<false, true> : (const void*)qtts::sh::qtts_shared_kernel<false, false>, qtts::sh::STHR, &a, &a.tag_base,
-                                      workspace, 1, sizeof(SWorkspace), stream);
+  const void* fn = a.sel.do_sample ? (const void*)qtts::sh::qtts_shared_kernel<false, true>
+                                   : (const void*)qtts::sh::qtts_shared_kernel<false, false>;
+  return qtts_host::launch_persistent(fn, qtts::sh::STHR, &a, &a.tag_base, workspace, 1, sizeof(SWorkspace), stream);
 }
 
 }  // extern "C"
