@@ -45,12 +45,10 @@ def _compare(bb, orc, p0, S, hidden, hidden_ref, label, bars=(TOL, TOL, TOL)):
 
 @pytest.mark.parametrize("S", [1, 7, 64, 128, 130, 256, 333, 1100])
 def test_prefill_two_layers(pkg, small, S):
-    """Prompt lengths across the tile edges and GEMM forms: one token and 7 (a partial 32-query
-    block; the row GEMM's partial 16-row block), 64 (two query blocks; 4 whole row blocks), 128
-    (the row GEMM's largest prompt, all 8 row blocks), 130 (the 64-column tile, a partial 128-row
-    tile), 256 (the smallest prompt of the DMA-fed 128 x 128 GEMM), several tiles with a ragged
-    last one, and a long prompt (the widest split-K target, 35 query blocks, a ragged last
-    block)."""
+    """Prompt lengths in every tile range up to 1,100 tokens (the edges are in test_gpu_prefill_tiles.py): one
+    token and 7 (a partial 32-query block, tiles mostly of rows past the prompt), 64 (two query blocks), 128 and
+    256 (the last lengths of their tiles), 130 and 333 (a ragged last row tile), and 1,100 (the largest
+    tiles, 35 query blocks, the last one ragged)."""
     dsd, tw = small
     ms = 512 if S <= 512 else 2048
     bb = pkg.TTSMegakernelGenerator(model=dsd, max_seq_len=ms)
@@ -69,8 +67,8 @@ def test_prefill_two_layers(pkg, small, S):
 @pytest.mark.parametrize("S", [100, 1100])
 def test_prefill_after_prefix_and_distinct_mrope(pkg, small, S):
     """A prompt continuing a cached prefix (positions 50..50 + S - 1 attend 0..50 + S - 1) with
-    distinct (t, h, w) rotary rows per token. At 1100 tokens the QKV GEMM is unsplit on 128-column
-    tiles and finishes each head (q/k-norm, RoPE, K/V write) in its own epilogue."""
+    distinct (t, h, w) rotary rows per token, on the smallest and the largest tiles of the QKV
+    projection, whose epilogue does q/k-norm, RoPE and the K/V write."""
     dsd, tw = small
     p0 = 50
     ms = 512 if p0 + S <= 512 else 2048
@@ -230,8 +228,8 @@ def test_prefill_then_decode_handoff(pkg, small):
 def test_prefill_fills_the_cache_in_one_or_two_calls(pkg, small):
     """Maximum size: a 4096-token prompt fills the whole cache (max_seq_len 4096) in one call,
     and again as two 2048-token calls, the second continuing from the first one's cache. Causal
-    attention makes the two equivalent; they differ only in summation order (the GEMMs split K
-    differently at 4096 and 2048 rows), so K, V and the last hidden agree within TOL. (The
+    attention makes the two equivalent; they differ only in summation order (the projections take
+    other tiles at 4096 and 2048 rows), so K, V and the last hidden agree within TOL. (The
     oracle is too slow at this size; the 2-layer cases above pin the arithmetic.)"""
     dsd, _ = small
     S = 4096

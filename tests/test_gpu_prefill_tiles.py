@@ -1,8 +1,9 @@
-"""The prefill at the prompt lengths where its tile and attention choices change, against a plain PyTorch
-float64 forward of the same two layers (no rounding between the operations): every K and V entry of both
-layers (the second layer's depend on every row of the first one's attention and MLP) and the last token's
-hidden. Bound: the GPU rounds to bf16 (2^-9 relative) after about ten operations a layer, independent
-roundings of about half of that each; 2 layers measured 3 to 5e-3 in norm, the bound is 1e-2.
+"""The prefill at the prompt lengths where its tile and attention choices change (32, 128, 256, 512, 1024, 1760,
+2048, 2688 and 4096 tokens) and at odd ones between them, against a plain PyTorch float64 forward of the same
+two layers (no rounding between the operations): every K and V entry of both layers (the second layer's depend
+on every row of the first one's attention and MLP) and the last token's hidden. Bound: the GPU rounds to bf16
+(2^-9 relative) after about ten operations a layer, independent roundings of about half of that each; 2 layers
+measured 3 to 5e-3 in norm, the bound is 1e-2.
 """
 import math
 
