@@ -283,7 +283,8 @@ hipError_t qtts_backbone_step_streams(
  * group-0 token is selected from bf16(codec_head . hidden) as in generator.py:113-119 (suppress
  * mask when mask_tail, EOS removed when suppress_eos, greedy or sampled) into out_token; the
  * logits go to out_logits when not NULL. workspace: >= qtts_prefill_workspace_bytes(n_tokens,
- * vocab) bytes, 256-byte aligned (contents need no initialisation). */
+ * vocab) bytes, 256-byte aligned (contents need no initialisation). Weights and caches are copied
+ * to LDS 16 bytes at a time: they are 16-byte aligned, as hipMalloc and torch return them. */
 size_t qtts_prefill_workspace_bytes(int n_tokens, int vocab);
 hipError_t qtts_backbone_prefill(
     void* workspace, size_t workspace_bytes, const TTSLayerWeights* layer_weights, int num_layers,
